@@ -8,383 +8,345 @@
 //
 // Both are fp32 fma chains in a fixed order: the reference accumulates
 // acc = fma(a, b, acc) (NVRTC's default --fmad=true) with k ascending from 0
-// for h, and with r ascending from out's own value for the rank add.  Each
-// output here runs the same chain in one lane, so the bits are the
-// reference's; the tiling only decides which lane owns which outputs.
-// lora_down pads K to its 32-deep tiles with zero products; the only effect
-// of that padding is fma(0, 0, -0) = +0, reproduced by one extra fma when
-// K % 32 != 0.
+// for h, and with r ascending from out's own value for the rank add.
 //
-// The chains are VALU work (R fmas per output element of the rank add), so
-// both kernels are sized for VALU issue: operands staged through LDS
-// transposed (k- or r-major), read with 16-byte loads, many accumulators per
-// lane.
-#include <cstdlib>
-
+// gfx950's fp32 MFMAs compute exactly such chains: D[i][j] is C[i][j] updated
+// by one fma a k-slice, k ascending, each rounded once, denormals kept
+// (16x16x4 and 32x32x2 compared with chains of fmaf over random, denormal,
+// overflowing, signed-zero and non-finite operands: every bit the same).  So
+// the matrix cores give the reference's bits at twice the rate of v_fmac_f32
+// and with a fraction of its operand traffic.
+//
+// An operand fragment holds, in lane group g (16 lanes) of a 4-deep k-slice,
+// column k0 + g of the lane's row.  Tiles are staged in LDS row by row at a
+// pitch of 4 floats more than a multiple of 32, and read back one float a lane
+// (two slices a ds_read2_b32): 16 rows x 4 columns hit 64 distinct banks.
+// Reading 16 bytes a lane and exchanging registers between the groups instead
+// (v_permlane16_swap / v_permlane32_swap) costs the wave more issue slots
+// than it saves: with one or two waves a SIMD the kernels are bound by the
+// instructions beside the MFMAs.
+//
+// Columns past K (or ranks past R) are padded with x = 0, A = -1: the product
+// is -0, and fma adds it to any accumulator (-0 included) without a change.
+// The reference's own padding of K to 32-deep tiles is with zero products,
+// whose only effect is fma(0, 0, -0) = +0, reproduced by one extra fma when
+// K % 32 != 0.
 #include "device_common.hpp"
 #include "lora.hpp"
 
 namespace phi_dev {
 
+// Four consecutive columns c.. of a row of `cols`, as loaded (bf16: in .x and
+// .y); columns past the row's end are replaced by others of the row.  VEC: one
+// access (cols % 4 == 0, the address aligned to it).  Branch-free: under a
+// branch the compiler waits for each load before the next.
+template <bool B16, bool VEC>
+__device__ __forceinline__ uint4 load4(const char* __restrict__ row, int c, int cols) {
+    constexpr int E = B16 ? 2 : 4;
+    if (VEC) {
+        const char* p = row + (uint64_t)((uint32_t)min(c, cols - 4) * (uint64_t)E);
+        if (!B16) return *(const uint4*)p;
+        const uint2 u = *(const uint2*)p;
+        return make_uint4(u.x, u.y, 0u, 0u);
+    }
+    uint32_t e[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const char* p = row + (uint64_t)((uint32_t)min(c + i, cols - 1) * (uint64_t)E);
+        e[i] = B16 ? *(const uint16_t*)p : *(const uint32_t*)p;
+    }
+    return B16 ? make_uint4(e[0] | e[1] << 16, e[2] | e[3] << 16, 0u, 0u) : make_uint4(e[0], e[1], e[2], e[3]);
+}
+
+// load4's value in fp32, and the same with columns from `cols` on replaced.
+template <bool B16>
+__device__ __forceinline__ float4 value4(const uint4& v) {
+    if (B16)
+        return make_float4(bf16_to_f32(v.x & 0xffffu), bf16_to_f32(v.x >> 16), bf16_to_f32(v.y & 0xffffu),
+                           bf16_to_f32(v.y >> 16));
+    return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+}
+template <bool VEC>
+__device__ __forceinline__ float4 pad4(const float4& v, int c, int cols, float pad) {
+    const bool i0 = c < cols, i1 = VEC ? i0 : c + 1 < cols, i2 = VEC ? i0 : c + 2 < cols, i3 = VEC ? i0 : c + 3 < cols;
+    return make_float4(i0 ? v.x : pad, i1 ? v.y : pad, i2 ? v.z : pad, i3 ? v.w : pad);
+}
+
 // ---- lora_down: h [M, R] = x [M, K] . A [R, K]^T -------------------------
-// Main form (x rows 16-byte aligned, K % 64 == 0): a block owns 64 rows and
-// 4 LD_TR ranks, a wave LD_TR of the ranks and a lane one row.  Each 64-k
-// chunk of the rows' x and of the waves' A slices goes global -> registers ->
-// LDS, double-buffered with one barrier a chunk, the next chunk's global
-// loads in flight under the current chunk's fmas.  A lane reads its own row
-// of x (68-float pitch: 16-byte aligned rows, conflict-free 16-byte reads and
-// writes) and its wave's A values, which all the wave's lanes read at one
-// address (a broadcast).  Earlier the A values came through the scalar cache;
-// scalar loads complete out of order, so only a full wait covers them, and
-// each 8-k step waited on a batch that missed the scalar cache.  LD_TR = 2
-// by default (PHI_LORA_TR=1 or 4 as A/B switches).
-constexpr int LD_KC = 64, LD_XP = LD_KC + 4;
+// A wave owns 16 RT rows x 16 ranks as RT chains of 16x16x4 MFMAs, K / 4
+// links each.  A chain is serial by contract, so the smallest output tile of
+// a full-rate MFMA gives the shortest one (32 clocks a link of 4 columns,
+// 10.2 us at K = 3072).  A block is 4 waves, WR of them over the ranks: 16 RT
+// rows x 64 ranks reads x once where R > 32.
+//
+// With one wave a SIMD nothing hides a wave's own latencies, so they are laid
+// under its MFMAs by hand.  Both operands' 64-column chunks go global ->
+// registers (LD_AHEAD chunks ahead) -> LDS (three buffers) -> fragments.
+// While the MFMAs of chunk c run, pair by pair, the fragments of c + 1 are
+// read, c + 2 is written to LDS and c + 2 + LD_AHEAD fetched; one barrier a
+// chunk.  The scheduling barriers keep that order: left alone the compiler
+// gathers a chunk's MFMAs behind their own fragment reads.  4352 x 3072 x 64:
+// 36.3 us, where one row a lane on v_fmac_f32 took 82.6.
+constexpr int LD_KC = 64, LD_P = LD_KC + 4, LD_AHEAD = 6;
 
-// TR consecutive floats (a TR * 4-byte aligned address) to and from registers.
-template <int TR>
-__device__ __forceinline__ void load_tr(const float* __restrict__ p, float (&v)[TR]) {
-    if constexpr (TR == 4) {
-        const float4 t = *(const float4*)p;
-        v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
-    } else if constexpr (TR == 2) {
-        const float2 t = *(const float2*)p;
-        v[0] = t.x, v[1] = t.y;
-    } else {
-        v[0] = *p;
-    }
-}
-
-template <int TR>
-__device__ __forceinline__ void store_tr(float* p, const float (&v)[TR]) {
-    if constexpr (TR == 4) *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
-    else if constexpr (TR == 2) *(float2*)p = make_float2(v[0], v[1]);
-    else *p = v[0];
-}
-
-// 64 rows x 64 k of x into registers: lane t holds row t / 4, k 16 (t % 4)..+15.
-template <bool XB>
-__device__ __forceinline__ void fetch_x_tile(const void* __restrict__ x, int64_t ldx, int m0, int M, int k0,
-                                             float (&v)[16]) {
-    const int row = threadIdx.x >> 2, kk = (threadIdx.x & 3) * 16;
-    const int64_t off = (int64_t)min(m0 + row, M - 1) * ldx + k0 + kk;
-    if (XB) {
-        const uint4 a = *(const uint4*)((const uint16_t*)x + off), b = *(const uint4*)((const uint16_t*)x + off + 8);
-        const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            v[2 * i] = bf16_to_f32(w[i] & 0xffffu);
-            v[2 * i + 1] = bf16_to_f32(w[i] >> 16);
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const float4 t = *(const float4*)((const float*)x + off + 4 * q);
-            v[4 * q] = t.x, v[4 * q + 1] = t.y, v[4 * q + 2] = t.z, v[4 * q + 3] = t.w;
-        }
-    }
-}
-
-template <bool XB, int LD_TR>
-__global__ __launch_bounds__(256) void lora_down_rows_kernel(const void* __restrict__ x, int64_t ldx,
-                                                             const float* __restrict__ A, float* __restrict__ h,
-                                                             int M, int K, int R) {
-    __shared__ __align__(16) float sx[2][64 * LD_XP];
-    __shared__ __align__(16) float sa[2][4][LD_TR * LD_KC];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int m0 = blockIdx.x * 64;
-    const int rb = (blockIdx.y * 4 + wave) * LD_TR;
-    const bool live = rb < R;  // wave-uniform; a dead wave still stages x for the others
-    // The wave's A slice of a chunk (LD_TR ranks x 64 k, rank-major): lane l
-    // holds LD_TR consecutive k of rank l / LPR.  Ranks past R read rank R - 1.
-    constexpr int LPR = LD_KC / LD_TR;
-    const int at = lane / LPR, ak = (lane % LPR) * LD_TR;
-    const float* arow = A + (int64_t)min(rb + at, R - 1) * K + ak;
-    float acc[LD_TR];
-#pragma unroll
-    for (int t = 0; t < LD_TR; t++) acc[t] = 0.0f;
-    float xt[16], ta[LD_TR];
-    fetch_x_tile<XB>(x, ldx, m0, M, 0, xt);
-    load_tr<LD_TR>(arow, ta);
-    const int srow = threadIdx.x >> 2, skk = (threadIdx.x & 3) * 16;
-    for (int k0 = 0, buf = 0; k0 < K; k0 += LD_KC, buf ^= 1) {
-        float* st = sx[buf] + srow * LD_XP + skk;
-#pragma unroll
-        for (int q = 0; q < 4; q++) *(float4*)(st + 4 * q) = make_float4(xt[4 * q], xt[4 * q + 1], xt[4 * q + 2], xt[4 * q + 3]);
-        store_tr<LD_TR>(&sa[buf][wave][at * LD_KC + ak], ta);
-        __syncthreads();
-        if (k0 + LD_KC < K) {
-            fetch_x_tile<XB>(x, ldx, m0, M, k0 + LD_KC, xt);
-            load_tr<LD_TR>(arow + k0 + LD_KC, ta);
-        }
-        if (live) {
-            const float* xr = sx[buf] + lane * LD_XP;
-            const float* as = sa[buf][wave];
-#pragma unroll
-            for (int kk = 0; kk < LD_KC; kk += 8) {
-                const float4 x0 = *(const float4*)(xr + kk), x1 = *(const float4*)(xr + kk + 4);
-                const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-                float av[LD_TR][8];
-#pragma unroll
-                for (int t = 0; t < LD_TR; t++) {
-                    const float4 a0 = *(const float4*)(as + t * LD_KC + kk), a1 = *(const float4*)(as + t * LD_KC + kk + 4);
-                    av[t][0] = a0.x, av[t][1] = a0.y, av[t][2] = a0.z, av[t][3] = a0.w;
-                    av[t][4] = a1.x, av[t][5] = a1.y, av[t][6] = a1.z, av[t][7] = a1.w;
-                }
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-#pragma unroll
-                    for (int t = 0; t < LD_TR; t++) acc[t] = fmaf(xv[i], av[t][i], acc[t]);
-            }
-        }
-        // The buffer written next iteration was last read two iterations ago,
-        // before this iteration's barrier: one barrier per chunk suffices.
-    }
-    const int m = m0 + lane;
-    if (!live || m >= M) return;
-    const bool pad = (K % 32) != 0;
-#pragma unroll
-    for (int t = 0; t < LD_TR; t++)
-        if (rb + t < R) h[(int64_t)m * R + rb + t] = pad ? fmaf(0.0f, 0.0f, acc[t]) : acc[t];
-}
-
-// General form (any alignment and K): block of 32 rows x 32 ranks, 256 lanes
-// of 2 x 2 outputs, K staged 64 deep through LDS, the next chunk's global
-// loads issued before the current chunk's fmas.
-constexpr int LD_BM = 32, LD_BR = 32, LD_BK = 64, LD_P = LD_BM + 4;
-
-template <bool XB>
-__device__ __forceinline__ void lora_down_fetch(const void* __restrict__ x, int64_t ldx, const float* __restrict__ A,
-                                                int M, int K, int R, int m0, int r0, int k0, int tid, float (&vx)[8],
-                                                float (&va)[8]) {
-    const int row = tid >> 3, k = k0 + (tid & 7) * 8;
-    const int m = m0 + row, r = r0 + row;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const bool in = m < M && k + i < K;
-        if (XB) vx[i] = in ? bf16_to_f32(((const uint16_t*)x)[(int64_t)m * ldx + k + i]) : 0.0f;
-        else vx[i] = in ? ((const float*)x)[(int64_t)m * ldx + k + i] : 0.0f;
-        va[i] = (r < R && k + i < K) ? A[(int64_t)r * K + k + i] : 0.0f;
-    }
-}
-
-template <bool XB>
+template <bool XB, bool VEC, int WR, int RT>
 __global__ __launch_bounds__(256) void lora_down_kernel(const void* __restrict__ x, int64_t ldx,
-                                                        const float* __restrict__ A, float* __restrict__ h,
-                                                        int M, int K, int R) {
-    __shared__ __align__(16) float sx[LD_BK][LD_P];
-    __shared__ __align__(16) float sa[LD_BK][LD_P];
-    const int tid = threadIdx.x;
-    const int m0 = blockIdx.x * LD_BM, r0 = blockIdx.y * LD_BR;
-    const int tm = (tid & 15) * 2, tr = (tid >> 4) * 2;
-    const int srow = tid >> 3, skk = (tid & 7) * 8;
-    float acc[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
-    float vx[8], va[8];
-    lora_down_fetch<XB>(x, ldx, A, M, K, R, m0, r0, 0, tid, vx, va);
-    for (int k0 = 0; k0 < K; k0 += LD_BK) {
+                                                        const float* __restrict__ A, float* __restrict__ h, int M,
+                                                        int K, int R) {
+    constexpr int WM = 4 / WR, XS = RT * WM, BM = 16 * XS, BR = 16 * WR, NS = XS + WR, BUF = (BM + BR) * LD_P / 4;
+    __shared__ float4 lds4[3 * BUF];
+    const float* lds = (const float*)lds4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m0 = blockIdx.x * BM, r0 = blockIdx.y * BR;
+    const int wm = wave / WR, wr = wave % WR;
+
+    // Slot i of a thread: row tid / 16 + 16 i of the chunk's rows (x's, then
+    // A's; rows past the last repeat it), columns 4 (tid % 16)..+3.
+    constexpr int XE = XB ? 2 : 4;
+    const int srow = tid >> 4, sc = (tid & 15) * 4;
+    const char* src[NS];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            sx[skk + i][srow] = vx[i];
-            sa[skk + i][srow] = va[i];
-        }
-        __syncthreads();
-        if (k0 + LD_BK < K) lora_down_fetch<XB>(x, ldx, A, M, K, R, m0, r0, k0 + LD_BK, tid, vx, va);
-        const int kn = min(LD_BK, K - k0);
-        if (kn == LD_BK) {
+    for (int i = 0; i < NS; i++)
+        src[i] = i < XS ? (const char*)x + (int64_t)min(m0 + srow + 16 * i, M - 1) * ldx * XE
+                        : (const char*)(A + (int64_t)min(r0 + srow + 16 * (i - XS), R - 1) * K);
+    auto fetch = [&](int i, int k0) {
+        return i < XS ? load4<XB, VEC>(src[i], k0 + sc, K) : load4<false, VEC>(src[i], k0 + sc, K);
+    };
+    auto stage = [&](int i, int buf, int k0, const uint4& v) {
+        const float4 f = i < XS ? pad4<VEC>(value4<XB>(v), k0 + sc, K, 0.0f) : pad4<VEC>(value4<false>(v), k0 + sc, K, -1.0f);
+        lds4[buf + (srow + 16 * i) * (LD_P / 4) + (tid & 15)] = f;
+    };
+    const int fx = (16 * RT * wm + (lane & 15)) * LD_P + (lane >> 4);
+    const int fa = (BM + 16 * wr + (lane & 15)) * LD_P + (lane >> 4);
+    auto frag_pair = [&](int buf, int q, float (&vx)[RT][16], float (&va)[16]) {  // links q and q + 1 of a chunk
 #pragma unroll
-            for (int kk = 0; kk < LD_BK; kk++) {
-                const float2 xv = *(const float2*)&sx[kk][tm];
-                const float2 av = *(const float2*)&sa[kk][tr];
-                acc[0][0] = fmaf(xv.x, av.x, acc[0][0]);
-                acc[0][1] = fmaf(xv.x, av.y, acc[0][1]);
-                acc[1][0] = fmaf(xv.y, av.x, acc[1][0]);
-                acc[1][1] = fmaf(xv.y, av.y, acc[1][1]);
-            }
-        } else {
-            for (int kk = 0; kk < kn; kk++) {
-                const float2 xv = *(const float2*)&sx[kk][tm];
-                const float2 av = *(const float2*)&sa[kk][tr];
-                acc[0][0] = fmaf(xv.x, av.x, acc[0][0]);
-                acc[0][1] = fmaf(xv.x, av.y, acc[0][1]);
-                acc[1][0] = fmaf(xv.y, av.x, acc[1][0]);
-                acc[1][1] = fmaf(xv.y, av.y, acc[1][1]);
-            }
+        for (int e = 0; e < 2; e++) {
+            va[q + e] = lds[4 * buf + fa + 4 * (q + e)];
+#pragma unroll
+            for (int t = 0; t < RT; t++) vx[t][q + e] = lds[4 * buf + fx + 16 * t * LD_P + 4 * (q + e)];
         }
-        __syncthreads();
+    };
+    v4f acc[RT];
+#pragma unroll
+    for (int t = 0; t < RT; t++) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+    const int nch = (K + LD_KC - 1) / LD_KC;
+    uint4 ring[LD_AHEAD][NS];
+    float vx[2][RT][16], va[2][16];
+    uint4 first[2][NS];
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int i = 0; i < NS; i++) first[c][i] = fetch(i, c * LD_KC);
+#pragma unroll
+    for (int c = 2; c < 2 + LD_AHEAD; c++)
+#pragma unroll
+        for (int i = 0; i < NS; i++) ring[c % LD_AHEAD][i] = fetch(i, c * LD_KC);
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int i = 0; i < NS; i++) stage(i, c * BUF, c * LD_KC, first[c][i]);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 16; q += 2) frag_pair(0, q, vx[0], va[0]);
+    int rd = BUF, wr_at = 2 * BUF;  // LDS offsets (float4) of chunks c + 1 (read) and c + 2 (written)
+    // Chunks in pairs: one past K holds only padding, which leaves the
+    // accumulators as they are.
+    for (int c = 0; c < nch; c += LD_AHEAD) {
+#pragma unroll
+        for (int u = 0; u < LD_AHEAD; u++) {
+            if (u > 0 && u % 2 == 0 && c + u >= nch) break;
+            const int cc = c + u;
+#pragma unroll
+            for (int q = 0; q < 16; q += 2) {
+#pragma unroll
+                for (int e = 0; e < 2; e++)
+#pragma unroll
+                    for (int t = 0; t < RT; t++)
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u & 1][q + e], vx[u & 1][t][q + e], acc[t], 0, 0, 0);
+                frag_pair(rd, q, vx[(u + 1) & 1], va[(u + 1) & 1]);
+#pragma unroll
+                for (int i = q / 2; i < NS; i += 8) {
+                    stage(i, wr_at, (cc + 2) * LD_KC, ring[(u + 2) % LD_AHEAD][i]);
+                    ring[(u + 2) % LD_AHEAD][i] = fetch(i, (cc + 2 + LD_AHEAD) * LD_KC);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            rd = wr_at;
+            wr_at = wr_at == 2 * BUF ? 0 : wr_at + BUF;
+            __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
+    // Lane: row lane % 16 of each of its tiles, ranks 4 (lane / 16)..+3.
+    const int r = r0 + 16 * wr + 4 * (lane >> 4);
     const bool pad = (K % 32) != 0;
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int t = 0; t < RT; t++) {
+        const int m = m0 + 16 * (RT * wm + t) + (lane & 15);
+        if (m >= M) continue;
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int m = m0 + tm + i, r = r0 + tr + j;
-            if (m < M && r < R) h[(int64_t)m * R + r] = pad ? fmaf(0.0f, 0.0f, acc[i][j]) : acc[i][j];
-        }
+        for (int e = 0; e < 4; e++)
+            if (r + e < R) h[(int64_t)m * R + r + e] = pad ? fmaf(0.0f, 0.0f, acc[t][e]) : acc[t][e];
+    }
 }
 
 // ---- lora_rank_add: C [M, N] += h [M, R] . B [N, R]^T ---------------------
-// Block: 128 x 128 outputs, 256 lanes of 8 x 8 (rows ty*8.., columns
-// tx*4.. and 64 + tx*4..), R staged 32 deep, r-major with a 132-float pitch.
-constexpr int RA_BM = 128, RA_BN = 128, RA_BR = 32, RA_P = 132;
+// C's read and write alone take 60 us at 4352 x 12288 (7.2 TB/s) and the
+// MFMAs of 64 ranks 44; the kernel takes 93 (the chains on v_fmac_f32: 116).
+// The MFMAs of some waves run under the memory phases of others: so small
+// tiles and few registers (four waves a SIMD; with 32 x 128 outputs a wave and
+// two waves a SIMD the two phases took turns, 120 us).
+// Block: 64 x 128 outputs; wave: 32 rows x 64 columns as 2 x 4 16x16x4 MFMA
+// tiles, tile t of a row holding columns 4 j + t (j = lane % 16), so that a
+// lane's four tiles are four adjacent columns: every access of C is 16 bytes
+// a lane (bf16: 8), a 256-byte piece of a row a lane group.  h and B are staged
+// 32 ranks at a time, B's rows in tile order within each 64 (row n at (n % 4)
+// 16 + n / 4).
+constexpr int RA_BM = 64, RA_BN = 128, RA_RC = 32, RA_P = RA_RC + 4;
 
-// One rank of the update: acc[i][j] = fma(h[row i], b[col j], acc[i][j]).
-__device__ __forceinline__ void rank_step(const float* __restrict__ hr, const float* __restrict__ br, int ty, int tx,
-                                          float (&acc)[8][8]) {
-    const float4 h0 = *(const float4*)&hr[ty * 8], h1 = *(const float4*)&hr[ty * 8 + 4];
-    const float4 b0 = *(const float4*)&br[tx * 4], b1 = *(const float4*)&br[64 + tx * 4];
-    const float hv[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-    const float bv[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+// CV: C's rows allow four-column accesses (N % 4 == 0, 16- or 8-byte aligned).
+// RV: h's and B's rows allow four-rank accesses (R % 4 == 0, 16-byte aligned).
+template <bool CB, bool CV, bool RV>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void lora_rank_add_kernel(
+    const float* __restrict__ h, const float* __restrict__ B, void* __restrict__ C, int64_t ldc, int M, int N, int R) {
+    __shared__ __align__(16) float sh[RA_BM * RA_P], sb[RA_BN * RA_P];
+    constexpr int CE = CB ? 2 : 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // Blocks are dealt to the 8 XCDs in turn: give each XCD a contiguous run of
+    // blocks, rows first, so that its L2 serves B's panel and h again and again
+    // beside C's stream (92.7 us against 102.9 with columns first).
+    const int nblk = gridDim.x, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3, tiles_m = (M + RA_BM - 1) / RA_BM;
+    const int blk = xcd * (nblk >> 3) + min(xcd, nblk & 7) + idx;
+    const int m0 = blk % tiles_m * RA_BM, n0 = blk / tiles_m * RA_BN;
+    const int wm = 32 * (wave >> 1), wn = 64 * (wave & 1);
+    const int col = n0 + wn + 4 * (lane & 15), row0 = m0 + wm + 4 * (lane >> 4);
+    const int srow = tid >> 3, sc = (tid & 7) * 4;
+    const char* src[6];
 #pragma unroll
-    for (int i = 0; i < 8; i++)
+    for (int s = 0; s < 6; s++)
+        src[s] = (const char*)(s < 2 ? h + (int64_t)min(m0 + srow + 32 * s, M - 1) * R
+                                     : B + (int64_t)min(n0 + srow + 32 * (s - 2), N - 1) * R);
+    uint4 v[6];
 #pragma unroll
-        for (int j = 0; j < 8; j++) acc[i][j] = fmaf(hv[i], bv[j], acc[i][j]);
-}
-
-// VEC: C's rows are 16-byte (fp32) or 8-byte (bf16) aligned and N % 4 == 0,
-// so each lane moves its four adjacent columns as one access.  Four waves a
-// SIMD (at most 128 VGPRs; the LDS holds four blocks a CU): against three at
-// the 134 the compiler picks unasked, 123.1 -> 110.9 us at 4352 x 12288 x 64,
-// with 32 bytes of spill a lane outside the rank loop.
-template <bool CB, bool VEC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void lora_rank_add_kernel(const float* __restrict__ h, const float* __restrict__ B,
-                                                            void* __restrict__ C, int64_t ldc, int M, int N, int R) {
-    __shared__ __align__(16) float sh[RA_BR][RA_P];
-    __shared__ __align__(16) float sb[RA_BR][RA_P];
-    const int tid = threadIdx.x;
-    const int m0 = blockIdx.y * RA_BM, n0 = blockIdx.x * RA_BN;
-    const int ty = tid >> 4, tx = tid & 15;
-    float acc[8][8];
+    for (int s = 0; s < 6; s++) v[s] = load4<false, RV>(src[s], sc, R);
+    v4f acc[2][4];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const int m = m0 + ty * 8 + i;
-        if constexpr (VEC) {
-#pragma unroll
-            for (int g = 0; g < 2; g++) {
-                const int n = n0 + g * 64 + tx * 4;
-                float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (m < M && n < N) {
-                    if (CB) {
-                        const uint2 u = *(const uint2*)((const uint16_t*)C + (int64_t)m * ldc + n);
-                        v[0] = bf16_to_f32(u.x & 0xffffu);
-                        v[1] = bf16_to_f32(u.x >> 16);
-                        v[2] = bf16_to_f32(u.y & 0xffffu);
-                        v[3] = bf16_to_f32(u.y >> 16);
-                    } else {
-                        const float4 f = *(const float4*)((const float*)C + (int64_t)m * ldc + n);
-                        v[0] = f.x;
-                        v[1] = f.y;
-                        v[2] = f.z;
-                        v[3] = f.w;
-                    }
-                }
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[i][g * 4 + e] = v[e];
-            }
-            continue;
-        }
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int n = n0 + (j >> 2) * 64 + tx * 4 + (j & 3);
-            float v = 0.0f;
-            if (m < M && n < N) {
-                if (CB) v = bf16_to_f32(((const uint16_t*)C)[(int64_t)m * ldc + n]);
-                else v = ((const float*)C)[(int64_t)m * ldc + n];
-            }
-            acc[i][j] = v;
-        }
+        const int m = min(row0 + 16 * (i >> 2) + (i & 3), M - 1);
+        const float4 f = value4<CB>(load4<CB, CV>((const char*)C + (int64_t)m * ldc * CE, col, N));
+        acc[i >> 2][0][i & 3] = f.x, acc[i >> 2][1][i & 3] = f.y, acc[i >> 2][2][i & 3] = f.z, acc[i >> 2][3][i & 3] = f.w;
     }
-    // R % 4 == 0 with 16-byte aligned h and B: a lane's four ranks of a row
-    // are one 16-byte load (r < R then covers r + 3).
-    const bool r4 = (R & 3) == 0 && ((uintptr_t)h & 15) == 0 && ((uintptr_t)B & 15) == 0;
-    for (int r0 = 0; r0 < R; r0 += RA_BR) {
-        // 128 rows x 32 ranks of h and of B: lane t loads 4 consecutive ranks of
-        // rows t/8 + 32 s and stores them rank-major.
+    const int fh = (wm + (lane & 15)) * RA_P + (lane >> 4), fb = (wn + (lane & 15)) * RA_P + (lane >> 4);
+    for (int r0 = 0; r0 < R; r0 += RA_RC) {
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int row = (tid >> 3) + 32 * s, rr = (tid & 7) * 4, r = r0 + rr;
-            const int m = m0 + row, n = n0 + row;
-            if (r4) {
-                const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                const float4 hv = (m < M && r < R) ? *(const float4*)&h[(int64_t)m * R + r] : z;
-                const float4 bv = (n < N && r < R) ? *(const float4*)&B[(int64_t)n * R + r] : z;
-                sh[rr][row] = hv.x, sh[rr + 1][row] = hv.y, sh[rr + 2][row] = hv.z, sh[rr + 3][row] = hv.w;
-                sb[rr][row] = bv.x, sb[rr + 1][row] = bv.y, sb[rr + 2][row] = bv.z, sb[rr + 3][row] = bv.w;
-                continue;
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                sh[rr + i][row] = (m < M && r + i < R) ? h[(int64_t)m * R + r + i] : 0.0f;
-                sb[rr + i][row] = (n < N && r + i < R) ? B[(int64_t)n * R + r + i] : 0.0f;
-            }
+        for (int s = 0; s < 6; s++) {
+            const int row = srow + 32 * (s < 2 ? s : s - 2);
+            float* d = s < 2 ? &sh[row * RA_P + sc] : &sb[((row & 64) + (row & 3) * 16 + ((row & 63) >> 2)) * RA_P + sc];
+            *(float4*)d = pad4<RV>(value4<false>(v[s]), r0 + sc, R, s < 2 ? 0.0f : -1.0f);
         }
         __syncthreads();
-        const int rn = min(RA_BR, R - r0);
-        for (int r = 0; r < rn; r++) rank_step(sh[r], sb[r], ty, tx, acc);
+        if (r0 + RA_RC < R) {
+#pragma unroll
+            for (int s = 0; s < 6; s++) v[s] = load4<false, RV>(src[s], r0 + RA_RC + sc, R);
+        }
+        const int steps = (min(RA_RC, R - r0) + 7) / 8;  // 8 ranks a step
+        for (int q = 0; q < steps; q++) {
+            float th[2][2], tb[4][2];
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+#pragma unroll
+                for (int u = 0; u < 2; u++) th[u][e] = sh[fh + 16 * u * RA_P + 8 * q + 4 * e];
+#pragma unroll
+                for (int t = 0; t < 4; t++) tb[t][e] = sb[fb + 16 * t * RA_P + 8 * q + 4 * e];
+            }
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int t = 0; t < 4; t++)
+                        acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(th[u][e], tb[t][e], acc[u][t], 0, 0, 0);
+        }
         __syncthreads();
     }
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const int m = m0 + ty * 8 + i;
+        const int m = row0 + 16 * (i >> 2) + (i & 3);
         if (m >= M) continue;
-        if constexpr (VEC) {
-#pragma unroll
-            for (int g = 0; g < 2; g++) {
-                const int n = n0 + g * 64 + tx * 4;
-                if (n >= N) continue;
-                const float* a = &acc[i][g * 4];
-                if (CB)
-                    *(uint2*)((uint16_t*)C + (int64_t)m * ldc + n) = make_uint2(f32x2_to_bf16x2(a[0], a[1]),
-                                                                                f32x2_to_bf16x2(a[2], a[3]));
-                else
-                    *(float4*)((float*)C + (int64_t)m * ldc + n) = make_float4(a[0], a[1], a[2], a[3]);
-            }
+        const float f[4] = {acc[i >> 2][0][i & 3], acc[i >> 2][1][i & 3], acc[i >> 2][2][i & 3], acc[i >> 2][3][i & 3]};
+        const int64_t off = (int64_t)m * ldc + col;
+        if (CV) {
+            if (col >= N) continue;
+            if (CB) *(uint2*)((uint16_t*)C + off) = make_uint2(f32x2_to_bf16x2(f[0], f[1]), f32x2_to_bf16x2(f[2], f[3]));
+            else *(float4*)((float*)C + off) = make_float4(f[0], f[1], f[2], f[3]);
             continue;
         }
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int n = n0 + (j >> 2) * 64 + tx * 4 + (j & 3);
-            if (n >= N) continue;
-            if (CB) ((uint16_t*)C)[(int64_t)m * ldc + n] = (uint16_t)f32_to_bf16(acc[i][j]);
-            else ((float*)C)[(int64_t)m * ldc + n] = acc[i][j];
+        for (int t = 0; t < 4; t++) {
+            if (col + t >= N) continue;
+            if (CB) ((uint16_t*)C)[off + t] = (uint16_t)f32_to_bf16(f[t]);
+            else ((float*)C)[off + t] = f[t];
         }
     }
 }
 
-template <int TR>
-static hipError_t launch_down_rows(hipStream_t stream, const void* x, bool x_bf16, int64_t ldx, const float* A,
-                                   float* h, int M, int K, int R) {
-    const dim3 grid((unsigned)((M + 63) / 64), (unsigned)((R + 4 * TR - 1) / (4 * TR)));
-    if (x_bf16) hipLaunchKernelGGL((lora_down_rows_kernel<true, TR>), grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
-    else hipLaunchKernelGGL((lora_down_rows_kernel<false, TR>), grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
+template <bool XB, bool VEC, int WR, int RT>
+static hipError_t launch_down(hipStream_t stream, const void* x, int64_t ldx, const float* A, float* h, int M, int K,
+                              int R) {
+    constexpr int BM = 16 * RT * (4 / WR), BR = 16 * WR;
+    const dim3 grid((unsigned)((M + BM - 1) / BM), (unsigned)((R + BR - 1) / BR));
+    hipLaunchKernelGGL((lora_down_kernel<XB, VEC, WR, RT>), grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
     return hipGetLastError();
+}
+
+// Waves over the ranks: as many 16-rank tiles as R has, up to four, so that no
+// wave of a block idles and x is read as few times as possible.  One chain a
+// wave while every chain finds a SIMD of its own (4 a CU), two beyond: the
+// pair takes as long as two chains on one SIMD would, and A is read half as
+// often.
+template <bool XB, bool VEC>
+static hipError_t launch_down_r(hipStream_t stream, const void* x, int64_t ldx, const float* A, float* h, int M, int K,
+                                int R) {
+    const bool one = ((int64_t)M + 15) / 16 * ((R + 15) / 16) <= 1024;
+    if (R <= 16) return one ? launch_down<XB, VEC, 1, 1>(stream, x, ldx, A, h, M, K, R)
+                            : launch_down<XB, VEC, 1, 2>(stream, x, ldx, A, h, M, K, R);
+    if (R <= 32) return one ? launch_down<XB, VEC, 2, 1>(stream, x, ldx, A, h, M, K, R)
+                            : launch_down<XB, VEC, 2, 2>(stream, x, ldx, A, h, M, K, R);
+    return one ? launch_down<XB, VEC, 4, 1>(stream, x, ldx, A, h, M, K, R)
+               : launch_down<XB, VEC, 4, 2>(stream, x, ldx, A, h, M, K, R);
 }
 
 hipError_t launch_lora_down(hipStream_t stream, const void* x, bool x_bf16, int64_t ldx, const float* A, float* h,
                             int M, int K, int R) {
     const int esz = x_bf16 ? 2 : 4;
-    if (K % LD_KC == 0 && (uintptr_t)x % 16 == 0 && (ldx * esz) % 16 == 0 && (uintptr_t)A % 16 == 0) {
-        const int tr = env_switch("PHI_LORA_TR", 2, 1, 4);  // A/B switch: ranks per wave (1, 2 or 4)
-        if (tr == 1) return launch_down_rows<1>(stream, x, x_bf16, ldx, A, h, M, K, R);
-        if (tr == 2) return launch_down_rows<2>(stream, x, x_bf16, ldx, A, h, M, K, R);
-        return launch_down_rows<4>(stream, x, x_bf16, ldx, A, h, M, K, R);
-    }
-    const dim3 grid((unsigned)((M + LD_BM - 1) / LD_BM), (unsigned)((R + LD_BR - 1) / LD_BR));
-    if (x_bf16) hipLaunchKernelGGL(lora_down_kernel<true>, grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
-    else hipLaunchKernelGGL(lora_down_kernel<false>, grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
+    const bool vec = K % 4 == 0 && ldx % 4 == 0 && (uintptr_t)x % (4 * esz) == 0 && (uintptr_t)A % 16 == 0;
+    if (x_bf16) return vec ? launch_down_r<true, true>(stream, x, ldx, A, h, M, K, R)
+                           : launch_down_r<true, false>(stream, x, ldx, A, h, M, K, R);
+    return vec ? launch_down_r<false, true>(stream, x, ldx, A, h, M, K, R)
+               : launch_down_r<false, false>(stream, x, ldx, A, h, M, K, R);
+}
+
+template <bool CB, bool CV>
+static hipError_t launch_add(hipStream_t stream, const float* h, const float* B, void* C, int64_t ldc, int M, int N,
+                             int R) {
+    const int64_t blocks = (int64_t)((N + RA_BN - 1) / RA_BN) * ((M + RA_BM - 1) / RA_BM);
+    if (blocks > INT32_MAX) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)blocks);
+    if (R % 4 == 0 && (uintptr_t)h % 16 == 0 && (uintptr_t)B % 16 == 0)
+        hipLaunchKernelGGL((lora_rank_add_kernel<CB, CV, true>), grid, dim3(256), 0, stream, h, B, C, ldc, M, N, R);
+    else
+        hipLaunchKernelGGL((lora_rank_add_kernel<CB, CV, false>), grid, dim3(256), 0, stream, h, B, C, ldc, M, N, R);
     return hipGetLastError();
 }
 
 hipError_t launch_lora_rank_add(hipStream_t stream, const float* h, const float* B, void* C, bool c_bf16, int64_t ldc,
                                 int M, int N, int R) {
-    const dim3 grid((unsigned)((N + RA_BN - 1) / RA_BN), (unsigned)((M + RA_BM - 1) / RA_BM));
     const bool vec = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (c_bf16 ? 8 : 16) == 0;
-    if (c_bf16) {
-        if (vec) hipLaunchKernelGGL((lora_rank_add_kernel<true, true>), grid, dim3(256), 0, stream, h, B, C, ldc, M, N, R);
-        else hipLaunchKernelGGL((lora_rank_add_kernel<true, false>), grid, dim3(256), 0, stream, h, B, C, ldc, M, N, R);
-    } else {
-        if (vec) hipLaunchKernelGGL((lora_rank_add_kernel<false, true>), grid, dim3(256), 0, stream, h, B, C, ldc, M, N, R);
-        else hipLaunchKernelGGL((lora_rank_add_kernel<false, false>), grid, dim3(256), 0, stream, h, B, C, ldc, M, N, R);
-    }
-    return hipGetLastError();
+    if (c_bf16) return vec ? launch_add<true, true>(stream, h, B, C, ldc, M, N, R)
+                           : launch_add<true, false>(stream, h, B, C, ldc, M, N, R);
+    return vec ? launch_add<false, true>(stream, h, B, C, ldc, M, N, R)
+               : launch_add<false, false>(stream, h, B, C, ldc, M, N, R);
 }
 
 }  // namespace phi_dev

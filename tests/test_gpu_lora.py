@@ -138,3 +138,30 @@ def test_lora_down_both_forms_agree(dev, orc):
     torch.cuda.synchronize()
     assert np.array_equal(bits(h_vec), orc.lora_down(x[:, :K].numpy(), A.numpy()).view(np.int32))
     assert np.array_equal(bits(h_gen), orc.lora_down(x[:, 1:].contiguous().numpy(), A.numpy()).view(np.int32))
+
+
+@pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,K,N,R", [(15, 64, 4, 4), (17, 68, 128, 16), (64, 448, 132, 20), (65, 4, 124, 32),
+                                     (1031, 392, 260, 36), (2100, 260, 8, 130), (16400, 64, 12, 8)])
+def test_lora_tiles_bit_exact(dev, orc, cdt, M, K, N, R):
+    """Edges of the tiles: rows and ranks around 16 and 64, columns around 64
+    and 128, K around the 64-column chunks, one chain a wave and two (above
+    1024 16 x 16 tiles), with denormal, zero and negative-zero operands."""
+    x, A, B, out = factors(M, K, R, N, M + 7 * K + R)
+    x[0] *= 1e-38
+    x[-1] = -0.0
+    A[:, ::3] = 0.0
+    B[N // 2] = -0.0
+    out[-1] = -0.0
+    x, out = x.to(cdt), out.to(cdt)
+    y = out.to(dev)
+    h = torch.empty((M, R), dtype=torch.float32, device=dev)
+    Q.lora_tail(x.to(dev), A.to(dev), B.to(dev), y, h=h)
+    torch.cuda.synchronize()
+    hw = orc.lora_down(x.float().numpy(), A.numpy())
+    assert np.array_equal(bits(h), hw.view(np.int32))
+    want = orc.lora_rank_add(hw, B.numpy(), out.float().numpy())
+    if cdt == torch.float32:
+        assert np.array_equal(bits(y), want.view(np.int32))
+    else:
+        assert torch.equal(y.cpu().view(torch.int16), torch.from_numpy(want).to(torch.bfloat16).view(torch.int16))
