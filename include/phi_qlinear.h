@@ -246,6 +246,9 @@ int64_t phi_hip_big_tile_rows(int64_t M, int64_t N);
  *             and split do not apply, group_m does); PHI_PLAN_TILE_AUTO (0):
  *             the library's cost model picks
  *   reserved  0
+ * A problem too small to fill the chip with these tiles runs on a kernel of
+ * smaller ones with K split over a block's waves, unless the table has an
+ * entry for it that sets a field.
  * Every plan gives the same bits; only the time differs.  The table is
  * process-wide and thread-safe; the host layer's GemmTuneStore sweeps,
  * persists and loads it.  _set with plan NULL removes the shape's entry;
@@ -339,7 +342,8 @@ phi_status phi_hip_w4a8_prepare(phi_stream_t stream, const phi_w4a8_weight* w, i
  *     registers.  Same bits on every path.
  *     The expand-once path and the LDS path (K <= 16384) keep the activation
  *     codes in the K-tiled layout (phi_hip_pack_k_tiled), so q8 then holds
- *     them K-tiled; s8 is the same on every path.
+ *     them K-tiled; s8 is the same on every path.  A problem too small for
+ *     either expands in registers, its codes read once, q8 row-major.
  */
 phi_status phi_hip_w4a8_linear(phi_stream_t stream, const void* x, int x_dtype, int64_t ldx,
                                int64_t M, int64_t K, const uint8_t* codes,

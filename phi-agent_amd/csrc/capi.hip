@@ -9,7 +9,9 @@
 // reported as PHI_ERR_DEVICE_LOST and stays sticky for the process.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -259,6 +261,58 @@ bool use_t272(const phi_dev::GemmParams& p, int G, int tile) {
     return t < square_plan_cost(p.M, p.N, G) - 1e-9;
 }
 
+// Below what a problem takes on the persistent kernels, in us: its rounds of
+// tiles at the fastest K-step measured (a round of 128 x 128 tiles with most
+// CUs idle; W4 codes expanded in registers: a full round of 256 x 256), one
+// pass over the operands, and the launch.
+double persist_us(const phi_dev::GemmParams& p, bool w4, int G) {
+    double rounds = square_plan_cost(p.M, p.N, G);
+    if (!w4 && phi_dev::t272_ok(p))
+        rounds = std::min(rounds, (p.kt ? (p.b_rm ? kT272RoundMixed : kT272Round) : kT272RoundRowMajor) *
+                                      (double)((phi_dev::t272_tile_count(p.M, p.N) + G - 1) / G));
+    const double steps = rounds * (p.K / 64), mb = ((double)p.N + p.M) * p.K / 1e6;
+    if (w4) return 4.0 + 1.05 * steps;
+    return p.kt ? 3.6 + 0.42 * steps + 0.15 * mb : 3.6 + 0.45 * steps + 0.20 * mb;
+}
+
+// The same of the register-staged tile kernels (gemm_kernel_for, gemm_cfg_for).
+double tile_us(const phi_dev::GemmParams& p, int G) {
+    const double t256 = ceil(p.M / 256.0) * ceil(p.N / 256.0);
+    const double small = ceil(p.M / 128.0) * ceil(p.N / 128.0);
+    const double rounds = t256 < 128 ? 0.40 * fmax(1.0, small / (2 * G)) : ceil(t256 / G);
+    return 4.0 + rounds * ((p.K + 63) / 64);
+}
+
+// The same of W4A8 with per-group tables: expanded once into a workspace, in
+// LDS on the 272 x 192 pipeline, or in registers.
+double w4a8_us(const phi_dev::GemmParams& p, int G, bool workspace) {
+    phi_dev::GemmParams q = p;
+    q.kt = 1;
+    if (workspace) return persist_us(q, false, G) + 0.30 * (double)p.N * p.K / 1e6;
+    if (p.K > 16384 || !phi_dev::t272w4_ok(q)) return persist_us(p, true, G);
+    return 4.0 + 0.7 * ceil((double)phi_dev::t272_tile_count(p.M, p.N) / G) * (p.K / 64);
+}
+
+// The small-problem kernel's tile for p where the model says it beats
+// `other_us`, or -1.  A kernel forced by an A/B switch keeps its problems;
+// PHI_GEMM_SKINNY=0..11 forces a tile of this one, any other value turns it
+// off.
+int skinny_choice(const phi_dev::GemmParams& p, bool w4, int G, double other_us) {
+    if (!phi_dev::skinny_ok(p, w4)) return -1;
+    if (getenv("PHI_GEMM_KERNEL") || getenv("PHI_GEMM_PIPE") || getenv("PHI_GEMM_MIXED") || getenv("PHI_GEMM_T272")) return -1;
+    if (getenv("PHI_GEMM_SKINNY")) return phi_dev::env_switch("PHI_GEMM_SKINNY", -1, 0, phi_dev::skinny_configs() - 1);
+    // The margin is the model's error: over 150 random shapes nothing it takes
+    // got slower, and half got more than 2.2 times faster (one row on 3072 ->
+    // 3072: 12.5 -> 4.6 us, 4096 rows onto 64 columns: 11.5 -> 4.8).
+    double us;
+    const int cfg = phi_dev::skinny_best(p, w4, G, &us);
+    return 1.15 * us + 0.5 < other_us ? cfg : -1;
+}
+
+// Whether a tuning-table entry says how the persistent kernel runs (and not
+// only the library's own choice, which may be the small-problem kernel).
+bool plan_is_set(const phi_gemm_plan& q) { return q.big_rows >= 0 || q.group_m > 0 || q.split || q.tile != PHI_PLAN_TILE_AUTO; }
+
 // The persistent kernel over the whole problem: 256 x 256 tiles for the rows
 // big_tile_rows() gives it (or the tuning table's plan), then 128 x 128 tiles
 // for the rest (A, sA, C and the output rows offset; B, sB and bias are shared);
@@ -269,6 +323,10 @@ hipError_t launch_persist_plan(hipStream_t stream, const phi_dev::GemmParams& p0
     const int64_t M = p0.M;
     phi_gemm_plan plan{};
     const bool tuned = gk == GK_PERSIST && !w4 && tuned_plan(M, p0.N, p0.K, p0.kt, &plan);
+    if (gk == GK_PERSIST && !(tuned && plan_is_set(plan))) {
+        const int cfg = skinny_choice(p0, w4, G, persist_us(p0, w4, G));
+        if (cfg >= 0) return phi_dev::launch_i8_gemm_skinny(stream, p0, w4, cfg);
+    }
     phi_dev::GemmParams p = p0;
     if (tuned && plan.group_m > 0) p.group_m = plan.group_m;
     if (gk == GK_PERSIST && !w4 && use_t272(p0, G, tuned ? plan.tile : PHI_PLAN_TILE_AUTO))
@@ -449,9 +507,14 @@ phi_status phi_hip_i8_gemm(phi_stream_t stream, const int8_t* A, int64_t lda, co
     p.c_kind = c_kind_of(c_dtype);
     p.group_m = 4;
     set_vec_flags(p, c_dtype, ldc);
+    const bool pok = persist_ok(C, c_dtype, N, K, lda, ldb, ldc);
+    if (staged_ok && !pok) {
+        const int cfg = skinny_choice(p, false, num_cus(), tile_us(p, num_cus()));
+        if (cfg >= 0) return check_hip(phi_dev::launch_i8_gemm_skinny((hipStream_t)stream, p, false, cfg), who);
+    }
     if (!staged_ok || (ek && strcmp(ek, "any") == 0))
         return check_hip(phi_dev::launch_i8_gemm_any((hipStream_t)stream, p, gemm_cfg_for(M, N)), who);
-    const GemmKernel gk = gemm_kernel_for(M, N, K, persist_ok(C, c_dtype, N, K, lda, ldb, ldc));
+    const GemmKernel gk = gemm_kernel_for(M, N, K, pok);
     if (gk == GK_PERSIST || gk == GK_PERSIST256 || gk == GK_PERSIST128)
         return check_hip(launch_persist_plan((hipStream_t)stream, p, gk, false, c_dtype, ldc), who);
     if (gk != GK_TILE128) {
@@ -762,6 +825,11 @@ phi_status phi_hip_q8_linear_kq(phi_stream_t stream, const void* x, int x_dtype,
         p.b_rm = 1;
         set_vec_flags(p, c_dtype, ldc);
         mixed = use_t272(p, num_cus(), PHI_PLAN_TILE_AUTO);
+        if (mixed) {  // the small-problem kernel, through phi_hip_q8_linear, where that beats it
+            phi_dev::GemmParams r = p;
+            r.kt = r.b_rm = 0;
+            mixed = skinny_choice(r, false, num_cus(), persist_us(p, false, num_cus())) < 0;
+        }
     }
     if (!mixed)
         return phi_hip_q8_linear(stream, x, x_dtype, ldx, M, K, W, ldw, sW, sw_scalar, bias, bias_dtype, N, C, c_dtype,
@@ -866,6 +934,31 @@ phi_status phi_hip_w4a8_linear(phi_stream_t stream, const void* x, int x_dtype, 
     // without a workspace it is the in-register path wherever it applies.
     // A kernel forced by PHI_GEMM_KERNEL keeps its own path.
     const int w4t = phi_dev::env_switch("PHI_W4_T272", -1, 0, 1);
+    phi_dev::GemmParams sp{};
+    sp.A = q8;
+    sp.B = (const int8_t*)codes;
+    sp.sA = s8;
+    sp.sB = s_w;
+    sp.bias = bias;
+    sp.C = C;
+    sp.lda = K;
+    sp.ldb = codes_row_bytes;
+    sp.ldc = ldc;
+    sp.M = (int)M;
+    sp.N = (int)N;
+    sp.K = (int)K;
+    sp.bias_kind = bk;
+    sp.c_kind = c_kind_of(c_dtype);
+    sp.lut = lut;
+    sp.lut_groups = K / group;
+    while ((1ll << sp.group_shift) < group) sp.group_shift++;
+    set_vec_flags(sp, c_dtype, ldc);
+    const int skinny = w4t < 0 ? skinny_choice(sp, true, num_cus(), w4a8_us(sp, num_cus(), workspace && need > 0 && ws_bytes >= need)) : -1;
+    if (skinny >= 0) {
+        st = phi_hip_quant_rotate(stream, x, x_dtype, M, K, ldx, q8, K, s8, 127.0f, round_mode, 1);
+        if (st != PHI_OK) return st;
+        return check_hip(phi_dev::launch_i8_gemm_skinny((hipStream_t)stream, sp, true, skinny), who);
+    }
     if (!e && w4t != 0 && (w4t == 1 || !(need > 0 && workspace && ws_bytes >= need)) && K <= 16384 &&
         aligned(q8, 16) && aligned(codes, 16) && codes_row_bytes % 16 == 0 &&
         persist_ok(C, c_dtype, N, K, K, codes_row_bytes, ldc)) {

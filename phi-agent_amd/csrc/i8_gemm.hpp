@@ -88,6 +88,15 @@ hipError_t launch_i8_gemm_pipe_mixed(hipStream_t stream, const GemmParams& pb, c
 bool t272_ok(const GemmParams& p);
 int t272_tile_count(int64_t M, int64_t N);
 hipError_t launch_i8_gemm_t272(hipStream_t stream, const GemmParams& p, int num_cus);
+// Problems too small to fill the chip with those tiles (i8_gemm_skinny.hip):
+// small tiles, K split over a block's waves.  Row-major or K-tiled operands,
+// or W4 codes (w4, with p.lut or p.w4_signed), any N and ldc, a gate with fp32
+// output (skinny_ok).  skinny_best: the fastest of its tiles for p by the
+// measured model, and its time; skinny_configs: how many there are.
+bool skinny_ok(const GemmParams& p, bool w4);
+int skinny_configs();
+int skinny_best(const GemmParams& p, bool w4, int num_cus, double* us);
+hipError_t launch_i8_gemm_skinny(hipStream_t stream, const GemmParams& p, bool w4, int cfg);
 // The same tiles with B as W4 codes (p.B [N, ldb], p.lut, p.group_shift)
 // expanded in LDS; K-tiled A, K % 1024 == 0 (t272w4_ok).
 bool t272w4_ok(const GemmParams& p);

@@ -1,0 +1,412 @@
+// int8 x int8 -> int32 GEMM for problems too small to fill the chip with
+// 128 x 128 tiles: few rows, few columns, or both (a prompt's or a small
+// image's tokens, a single row, the projection onto a few channels).  Same
+// product and epilogue as the persistent kernels (core/kernels/int8_gemm.cpp:
+// 466-621, epilogue :588-620; host gemm_int8 core/host/quant.cpp:223-236):
+//   C[m,n] = fma((float)acc[m,n] * sA[m], sB[n], bias[n]), or with a gate
+//   C[m,n] = fma(that, gate[n], C[m,n]) on fp32 C.
+//
+// What bounds such a problem is one pass over the weight, and latency: at one
+// row the weight's bytes are all the traffic there is.  A 128 x 128 tile walks
+// K alone on one CU (3072 -> 3072 has 24 of them, 11.9 us at one row on 24 of
+// 256 CUs).  Here a block owns a small tile, (16 MT) x (16 NT) outputs, and
+// its NW waves split K: wave w takes the 128-column pairs w, w + NW, ... The
+// int32 partial sums are exact in any order and meet in LDS.  That needs no
+// workspace and no second launch, and the tile can be as small as the shape
+// wants: 192 blocks of 16 waves for the example.
+//
+// A wave streams its operands through LDS of its own (no barriers): the
+// 16-byte chunks of a 128-column pair by direct-to-LDS loads, whole 128-byte
+// lines of 8 rows (row-major) or 1 KB of a K-tiled block an instruction, then
+// 16-byte fragment reads.  Loading the fragments straight into registers puts
+// 16 different rows into each 16-lane quarter of a load, 64 line accesses an
+// instruction, and ran at 16 bytes a clock and CU (31 K-tiled).  In a pair
+// lane group g (16 lanes) multiplies columns 32 g .. +31 as two fragments
+// (the sum over k may take them in any order, if A and B agree): packed 4-bit
+// weights are the same 32 columns in one 16-byte read, expanded in registers.
+#include <cmath>
+
+#include "device_common.hpp"
+#include "i8_gemm.hpp"
+#include "persist_common.hpp"
+
+namespace phi_dev {
+
+using persist::u32x4;
+
+enum SkinnyB { SB_I8 = 0, SB_LUT = 1, SB_S4 = 2 };
+
+typedef __attribute__((address_space(3))) int8_t lds_i8;
+
+// One operand's 16-row tile as the wave loads and reads it: a buffer resource
+// at the tile, the lane's byte offsets for a pair's two 1 KB loads, the bytes
+// from a pair to the next, and the offsets of the lane's two fragments in the
+// 2 KB the loads fill.
+struct Tile16 {
+    __amdgpu_buffer_rsrc_t rsrc;
+    int vo0, vo1, step, f0, f1;
+};
+
+// Rows r0.. of a row-major operand (pitch ld), or of a K-tiled one.  Rows past
+// the last read it again; their products are not stored.  Row-major: load j
+// fetches rows 8 j + l / 8, slot l % 8 of a row's 128 bytes holding chunk
+// slot ^ ((row >> 1) & 7), so that the fragment reads of 16 rows hit 16
+// distinct bank windows; K-tiled: load j is K-step j of the pair, swizzled in
+// memory already (k_tiled_offset).
+__device__ __forceinline__ Tile16 tile16(const int8_t* base, int64_t ld, bool kt, int r0, int rows, int K, int lane) {
+    Tile16 t;
+    const int r = lane & 15, g = lane >> 4, last = rows - 1 - r0;
+    if (!kt) {
+        t.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(base + (int64_t)r0 * ld), (short)0, 0x7fffffff, persist::kRsrcWord3);
+        const int ra = lane >> 3, rb = 8 + ra;
+        t.vo0 = min(ra, last) * (int)ld + (((lane & 7) ^ ((ra >> 1) & 7)) << 4);
+        t.vo1 = min(rb, last) * (int)ld + (((lane & 7) ^ ((rb >> 1) & 7)) << 4);
+        t.step = 128;
+        t.f0 = r * 128 + (((2 * g) ^ ((r >> 1) & 7)) << 4);
+        t.f1 = r * 128 + (((2 * g + 1) ^ ((r >> 1) & 7)) << 4);
+    } else {
+        const int s = r0 >> 8, rr = r0 & 255, h = min(256, rows - (s << 8));
+        t.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(base + (int64_t)s * 256 * K + rr * 64), (short)0, 0x7fffffff,
+                                                   persist::kRsrcWord3);
+        t.vo0 = min(lane >> 2, last) * 64 + (lane & 3) * 16;
+        t.vo1 = t.vo0 + h * 64;
+        t.step = h * 128;
+        const int x = (r >> 2) & 3, c = (2 * g) & 3, at = (g >> 1) * 1024 + r * 64;
+        t.f0 = at + ((c ^ x) << 4);
+        t.f1 = at + (((c + 1) ^ x) << 4);
+    }
+    return t;
+}
+
+// 32 signed nibbles (16 bytes, column order) as two fragments of int8 values
+// times 16: a nibble in the high half of a byte is its signed value times 16.
+// The sums come out times 16 exactly and are shifted back (K <= 65536 keeps
+// them in 32 bits).
+__device__ __forceinline__ void expand_s4(const u32x4& c, v4i& f0, v4i& f1) {
+    uint32_t o[8];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t even = (c[i] << 4) & 0xf0f0f0f0u, odd = c[i] & 0xf0f0f0f0u;
+        o[2 * i] = __builtin_amdgcn_perm(odd, even, 0x05010400u);
+        o[2 * i + 1] = __builtin_amdgcn_perm(odd, even, 0x07030602u);
+    }
+    f0 = v4i{(int)o[0], (int)o[1], (int)o[2], (int)o[3]};
+    f1 = v4i{(int)o[4], (int)o[5], (int)o[6], (int)o[7]};
+}
+
+// Bytes of a wave's stage (one pair of its tile's rows), and its loads.
+template <int MT, int NT, int SB>
+constexpr int skinny_stage = MT * 2048 + NT * (SB == SB_I8 ? 2048 : SB == SB_S4 ? 1024 : 1536);
+template <int MT, int NT, int SB>
+constexpr int skinny_loads = 2 * MT + (SB == SB_S4 ? 1 : 2) * NT;
+
+// A wave's LDS: its stages, and after the last pair its partial sums.
+template <int MT, int NT, int S, int SB>
+constexpr int skinny_region = S * skinny_stage<MT, NT, SB> > MT * NT * 1024 ? S * skinny_stage<MT, NT, SB> : MT * NT * 1024;
+
+template <int MT, int NT, int NW, int S, int SB>
+__device__ __forceinline__ void skinny_tile(const GemmParams& p, int8_t* smem) {
+    constexpr int BM = 16 * MT, BN = 16 * NT, T = MT * NT, STG = skinny_stage<MT, NT, SB>, D = skinny_loads<MT, NT, SB>;
+    constexpr int REG = skinny_region<MT, NT, S, SB>;
+    static_assert((S - 1) * D < 64, "vmcnt is six bits");
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // Each XCD takes a contiguous run of blocks, rows first: the blocks that
+    // read one panel of the weight run together on one L2.
+    const int tiles_m = (p.M + BM - 1) / BM;
+    const int blk = persist::xcd_remap(blockIdx.x, gridDim.x);
+    const int m0 = blk % tiles_m * BM, n0 = blk / tiles_m * BN;
+    int8_t* ring = persist::opaque_lds(smem + wave * REG);
+
+    Tile16 a[MT], b[NT];
+    int tv[NT];  // SB_LUT: the lane's byte offset into the tables, group 0
+    const __amdgpu_buffer_rsrc_t rl = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(SB == SB_LUT ? p.lut + (int64_t)n0 * p.lut_groups * 16 : p.A), (short)0, 0x7fffffff, persist::kRsrcWord3);
+#pragma unroll
+    for (int i = 0; i < MT; i++) a[i] = tile16(p.A, p.lda, p.kt, min(m0 + 16 * i, p.M - 1), p.M, p.K, lane);
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const int r0 = min(n0 + 16 * j, p.N - 1), last = p.N - 1 - r0;
+        if (SB == SB_I8) {
+            b[j] = tile16(p.B, p.ldb, p.kt && !p.b_rm, r0, p.N, p.K, lane);
+        } else {
+            // 16 rows x 64 bytes of codes a load; chunk c of row r in slot c ^ ((r >> 2) & 3).
+            b[j].rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(p.B + (int64_t)r0 * p.ldb), (short)0, 0x7fffffff,
+                                                          persist::kRsrcWord3);
+            const int row = lane >> 2, r = lane & 15;
+            b[j].vo0 = min(row, last) * (int)p.ldb + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
+            b[j].f0 = r * 64 + ((g ^ ((r >> 2) & 3)) << 4);
+            tv[j] = (r0 - n0 + min(r, last)) * (int)p.lut_groups * 16;
+        }
+    }
+    // The tables of a pair: lane l < 32 loads the one of row l % 16 for columns
+    // 64 (l / 16).. of the pair (with groups of 128 and up, the same twice).
+    auto issue = [&](int st, int pair) {
+        int8_t* d = ring + st * STG;
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            if (SB == SB_I8) {
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(b[j].rsrc, (persist::lptr_t)(d + j * 2048), 16, b[j].vo0, pair * b[j].step, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(b[j].rsrc, (persist::lptr_t)(d + j * 2048 + 1024), 16, b[j].vo1, pair * b[j].step, 0, 0);
+            } else {
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(b[j].rsrc, (persist::lptr_t)(d + j * 1024), 16, b[j].vo0, pair * 64, 0, 0);
+            }
+        }
+        int8_t* da = d + STG - MT * 2048;
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(a[i].rsrc, (persist::lptr_t)(da + i * 2048), 16, a[i].vo0, pair * a[i].step, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(a[i].rsrc, (persist::lptr_t)(da + i * 2048 + 1024), 16, a[i].vo1, pair * a[i].step, 0, 0);
+        }
+        if (SB == SB_LUT && lane < 32) {
+            const int gi = (pair * 128 + (lane >> 4) * 64) >> p.group_shift;
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rl, (persist::lptr_t)(d + NT * 1024 + j * 512), 16, tv[j] + gi * 16, 0, 0, 0);
+        }
+    };
+
+    v4i acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = v4i{0, 0, 0, 0};
+    v4i fa[MT][2], fb[NT][2];
+    auto read = [&](int st) {
+        const int8_t* d = ring + st * STG;
+        const int8_t* da = d + STG - MT * 2048;
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            if (SB == SB_I8) {
+                fb[j][0] = *(const v4i*)(d + j * 2048 + b[j].f0);
+                fb[j][1] = *(const v4i*)(d + j * 2048 + b[j].f1);
+            } else {
+                fb[j][0] = *(const v4i*)(d + j * 1024 + b[j].f0);
+                if (SB == SB_LUT) fb[j][1] = *(const v4i*)(d + NT * 1024 + j * 512 + ((g >> 1) * 16 + (lane & 15)) * 16);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            fa[i][0] = *(const v4i*)(da + i * 2048 + a[i].f0);
+            fa[i][1] = *(const v4i*)(da + i * 2048 + a[i].f1);
+        }
+    };
+    auto multiply = [&] {
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            v4i w0 = fb[j][0], w1 = fb[j][1];
+            if (SB != SB_I8) {
+                const u32x4 c = __builtin_bit_cast(u32x4, fb[j][0]), t = __builtin_bit_cast(u32x4, fb[j][1]);
+                if (SB == SB_S4) {
+                    expand_s4(c, w0, w1);
+                } else {
+                    w0 = persist::expand16b(c[0], c[1], t);
+                    w1 = persist::expand16b(c[2], c[3], t);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0, fa[i][0], acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1, fa[i][1], acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+
+    // Pairs wave, wave + NW, ...: S of them in flight.  A pair's stage is
+    // refilled as soon as its fragments are in registers.
+    const int pairs = p.K >> 7, n = (pairs - wave + NW - 1) / NW;
+    for (int i = 0; i < S && i < n; i++) issue(i, wave + i * NW);
+    for (int i = 0, st = 0; i < n; i++) {
+        // Loads complete in order: stage i has landed when only the younger
+        // stages' loads are left.
+        const int young = min(S - 1, n - 1 - i);
+        __builtin_amdgcn_sched_barrier(0);
+        if (S > 3 && young >= 3) persist::wait_vm_lgkm0<(S > 3 ? 3 * D : 0)>();
+        else if (S > 2 && young == 2) persist::wait_vm_lgkm0<(S > 2 ? 2 * D : 0)>();
+        else if (S > 1 && young == 1) persist::wait_vm_lgkm0<(S > 1 ? D : 0)>();
+        else persist::wait_vm_lgkm0<0>();
+        __builtin_amdgcn_sched_barrier(0);
+        read(st);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0): the fragments are read
+        if (i + S < n) issue(st, wave + (i + S) * NW);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply();
+        st = st + 1 == S ? 0 : st + 1;
+    }
+
+    // The wave's partial sums into its own stages (its loads and reads are
+    // over), then the block's sum.
+    __builtin_amdgcn_sched_barrier(0);
+    v4i* mine = (v4i*)ring;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) mine[(i * NT + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+
+    // Lane l of tile (i, j): row 16 i + l % 16, columns 16 j + 4 (l / 16)..+3.
+    for (int e = tid; e < T * 64; e += NW * 64) {
+        const int8_t* part = persist::opaque_lds(smem) + e * 16;
+        v4i s = *(const v4i*)part;
+#pragma unroll
+        for (int w = 1; w < NW; w++) s += *(const v4i*)(part + w * REG);
+        if (SB == SB_S4) s >>= 4;
+        const int tile = e >> 6, l = e & 63;
+        const int m = m0 + 16 * (tile / NT) + (l & 15), nn = n0 + 16 * (tile % NT) + 4 * (l >> 4);
+        if (m >= p.M || nn >= p.N) continue;
+        const int64_t off = (int64_t)m * p.ldc + nn;
+        const bool whole = p.c_vec && nn + 4 <= p.N;
+        if (p.c_kind == C_I32) {
+            int32_t* C = (int32_t*)p.C + off;
+            if (whole) {
+                *(v4i*)C = s;
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (nn + k < p.N) C[k] = s[k];
+            }
+            continue;
+        }
+        const float sa = p.sA[m];
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int nk = min(nn + k, p.N - 1);
+            const float sb = p.sB[p.sb_scalar ? 0 : nk];
+            float bz = 0.0f;
+            if (p.bias_kind == BIAS_F32) bz = ((const float*)p.bias)[nk];
+            else if (p.bias_kind == BIAS_BF16) bz = bf16_to_f32(((const uint16_t*)p.bias)[nk]);
+            v[k] = fmaf((float)s[k] * sa, sb, bz);
+        }
+        if (p.c_kind == C_BF16) {
+            uint16_t* C = (uint16_t*)p.C + off;
+            if (whole) {
+                *(uint2*)C = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (nn + k < p.N) C[k] = (uint16_t)f32_to_bf16(v[k]);
+            }
+            continue;
+        }
+        float* C = (float*)p.C + off;
+        if (p.gate) {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (nn + k < p.N) C[k] = fmaf(v[k], p.gate[nn + k], C[k]);
+        } else if (whole) {
+            *(float4*)C = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (nn + k < p.N) C[k] = v[k];
+        }
+    }
+}
+
+// The tiles the kernel is built for: wave tile, waves a block, stages a wave.
+// More waves beat more stages a wave (4 x 4 tiles over K = 12288 at 256 rows:
+// 26.3 us with 8 waves of one stage, 27.0 with 4 of two).
+struct SkinnyCfg {
+    int mt, nt, nw, s;
+};
+constexpr SkinnyCfg kSkinny[] = {{1, 1, 8, 2}, {1, 2, 8, 1}, {1, 4, 8, 1}, {2, 1, 8, 1}, {2, 2, 8, 1}, {2, 4, 8, 1},
+                                 {4, 1, 8, 1}, {4, 2, 8, 1}, {4, 4, 8, 1}, {5, 2, 8, 1}, {5, 4, 8, 1}, {6, 4, 4, 2}};
+constexpr int kSkinnyCfgs = (int)(sizeof kSkinny / sizeof kSkinny[0]);
+
+int skinny_configs() { return kSkinnyCfgs; }
+
+// Time of p on tile cfg in us: a fixed part, then the larger of the weight's
+// one pass from memory and the busiest CU's blocks, each its operands' bytes
+// at a CU's rate into LDS plus a part that grows with the tile (the fill, the
+// sum over waves, the stores).  Fitted over 90 shapes x 12 tiles (one to 2048
+// rows, 64 to 12288 columns, K 1024 to 12288, both layouts; rms error 15 %):
+// the tile it picks is within 1 % of the best on average, 12 % at worst.
+static double skinny_us(const GemmParams& p, bool w4, int num_cus, int cfg) {
+    const SkinnyCfg c = kSkinny[cfg];
+    const double blocks = (double)((p.M + 16 * c.mt - 1) / (16 * c.mt)) * (double)((p.N + 16 * c.nt - 1) / (16 * c.nt));
+    const double rounds = ceil(blocks / num_cus), pairs = p.K / 128.0, weight = (double)p.N * p.K * (w4 ? 0.5 : 1.0);
+    const double kb = pairs * (2.0 * c.mt + (!w4 ? 2.0 : p.w4_signed ? 1.0 : 1.5) * c.nt);
+    if (w4 && !p.w4_signed)
+        return 2.6 + fmax(rounds * (kb * 0.0097 + pairs * c.nt * 0.027 + 0.180 * c.mt * c.nt), weight / 2.1e6);
+    if (w4) return 2.8 + fmax(rounds * (kb * 0.0080 + 0.234 * c.mt * c.nt + 0.11), weight / 5.6e6);
+    return 2.0 + fmax(rounds * (kb * 0.01326 + 0.139 * c.mt * c.nt + 0.16), weight / 4.1e6);
+}
+
+int skinny_best(const GemmParams& p, bool w4, int num_cus, double* us) {
+    int best = 0;
+    double t = 1e300;
+    for (int i = 0; i < kSkinnyCfgs; i++) {
+        const double ti = skinny_us(p, w4, num_cus, i);
+        if (ti < t) t = ti, best = i;
+    }
+    *us = t;
+    return best;
+}
+
+template <int MT, int NT, int NW, int S, int SB>
+__global__ __launch_bounds__(NW * 64) void i8_gemm_skinny_kernel(GemmParams p) {
+    extern __shared__ __align__(16) int8_t smem[];
+    skinny_tile<MT, NT, NW, S, SB>(p, smem);
+}
+
+template <int MT, int NT, int NW, int S, int SB>
+static hipError_t launch_one(hipStream_t stream, const GemmParams& p) {
+    const int64_t blocks = (int64_t)((p.M + 16 * MT - 1) / (16 * MT)) * ((p.N + 16 * NT - 1) / (16 * NT));
+    if (blocks > INT32_MAX) return hipErrorInvalidValue;
+    constexpr int lds = NW * skinny_region<MT, NT, S, SB>;
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute((const void*)i8_gemm_skinny_kernel<MT, NT, NW, S, SB>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((i8_gemm_skinny_kernel<MT, NT, NW, S, SB>), dim3((unsigned)blocks), dim3(NW * 64), lds, stream, p);
+    return hipGetLastError();
+}
+
+template <int MT, int NT, int NW, int S>
+static hipError_t launch_cfg(hipStream_t stream, const GemmParams& p, int sb) {
+    switch (sb) {
+        case SB_I8: return launch_one<MT, NT, NW, S, SB_I8>(stream, p);
+        case SB_LUT: return launch_one<MT, NT, NW, S, SB_LUT>(stream, p);
+        default: return launch_one<MT, NT, NW, S, SB_S4>(stream, p);
+    }
+}
+
+template <int I>
+static hipError_t launch_at(hipStream_t stream, const GemmParams& p, int sb) {
+    return launch_cfg<kSkinny[I].mt, kSkinny[I].nt, kSkinny[I].nw, kSkinny[I].s>(stream, p, sb);
+}
+
+hipError_t launch_i8_gemm_skinny(hipStream_t stream, const GemmParams& p, bool w4, int cfg) {
+    const int sb = !w4 ? SB_I8 : p.w4_signed ? SB_S4 : SB_LUT;
+    switch (cfg) {
+        case 0: return launch_at<0>(stream, p, sb);
+        case 1: return launch_at<1>(stream, p, sb);
+        case 2: return launch_at<2>(stream, p, sb);
+        case 3: return launch_at<3>(stream, p, sb);
+        case 4: return launch_at<4>(stream, p, sb);
+        case 5: return launch_at<5>(stream, p, sb);
+        case 6: return launch_at<6>(stream, p, sb);
+        case 7: return launch_at<7>(stream, p, sb);
+        case 8: return launch_at<8>(stream, p, sb);
+        case 9: return launch_at<9>(stream, p, sb);
+        case 10: return launch_at<10>(stream, p, sb);
+        default: return launch_at<11>(stream, p, sb);
+    }
+}
+
+// Whether the kernel takes p: whole 128-column pairs and 16-byte operand
+// chunks; signed nibbles times 16 within 32 bits.
+bool skinny_ok(const GemmParams& p, bool w4) {
+    auto al = [](const void* q, int64_t ld) { return (uintptr_t)q % 16 == 0 && ld % 16 == 0; };
+    if (p.K % 128 != 0 || !al(p.A, p.kt ? 16 : p.lda) || !al(p.B, p.kt && !p.b_rm ? 16 : p.ldb)) return false;
+    if (w4 && p.w4_signed && p.K > 65536) return false;
+    // 32-bit byte offsets within a tile's rows (at most 128) and along K.
+    const int64_t lim = (int64_t)1 << 23;
+    if (p.lda >= lim || p.ldb >= lim || p.K >= lim || p.lut_groups * 16 >= lim) return false;
+    return true;
+}
+
+}  // namespace phi_dev
