@@ -145,6 +145,8 @@ hipError_t launch_quant_rotate(hipStream_t stream, const void* x, bool bf16_in, 
                                float qmax, int half_even, int rotate, const QrPre& pre, int q_kt = 0);
 // An int8 [rows, ld] row-major matrix into the K-tiled layout (16-byte aligned rows).
 hipError_t launch_pack_k_tiled(hipStream_t stream, const int8_t* src, int64_t ld, int64_t rows, int64_t K, int8_t* dst);
+// The rotation alone (phi_hip_convrot_rows) for 16-byte aligned rows; y may be x.
+hipError_t launch_convrot_teams(hipStream_t stream, const float* x, int64_t ldx, float* y, int64_t ldy, int64_t rows, int64_t K);
 size_t quant_rotate_lds_bytes(int64_t K);
 
 }  // namespace phi_dev

@@ -784,6 +784,59 @@ hipError_t launch_quant_rotate(hipStream_t stream, const void* x, bool bf16_in, 
     return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------
+// The rotation alone, fp32 in and out (phi_hip_convrot_rows): a wave takes
+// four consecutive 256-groups of a row, one 16-lane team each, as the register
+// form above does, with its tiles and the reference's butterflies (multiply
+// and subtract).  y may be x: a team has read its group before it writes it.
+// 302 MB of traffic at 12288 x 3072: 58 us; one element a thread with eight
+// barriers took 108.
+__global__ __launch_bounds__(256) void convrot_teams_kernel(const float* x, int64_t ldx, float* y, int64_t ldy,
+                                                            int64_t groups, int gpr) {
+    __shared__ __align__(16) float lds[4 * QT_WAVE];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, team = lane >> 4, tl = lane & 15, sw = tl >> 2;
+    const int64_t at = ((int64_t)blockIdx.x * 4 + wave) * 4 + team, g = at < groups ? at : groups - 1;
+    const int64_t row = g / gpr, col = (g - row * gpr) * 256 + tl * 16;
+    float* T = lds + wave * QT_WAVE + team * QT_TILE;
+    float* trow = T + tl * 16;
+    float v[16], w[16];
+    load16<false>(x, row * ldx + col, v);
+    bfly16<1>(v);
+    bfly16<4>(v);
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+        *(float4*)(trow + 4 * (c ^ sw)) = make_float4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
+    wave_lds_fence();
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float* cp = T + 64 * k + 4 * (sw ^ k) + (tl & 3);
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[4 * k + i] = cp[16 * i];
+    }
+    wave_lds_fence();
+    bfly16<1>(w);
+    bfly16<4>(w);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        float* cp = T + 64 * k + 4 * (sw ^ k) + (tl & 3);
+#pragma unroll
+        for (int i = 0; i < 4; i++) cp[16 * i] = w[4 * k + i] * (1.0f / 16.0f);
+    }
+    wave_lds_fence();
+    if (at >= groups) return;
+    float4* dst = (float4*)(y + row * ldy + col);
+#pragma unroll
+    for (int k = 0; k < 4; k++) dst[k] = *(const float4*)(trow + 4 * (k ^ sw));
+}
+
+hipError_t launch_convrot_teams(hipStream_t stream, const float* x, int64_t ldx, float* y, int64_t ldy, int64_t rows,
+                                int64_t K) {
+    const int64_t groups = rows * (K / 256);
+    hipLaunchKernelGGL(convrot_teams_kernel, dim3((unsigned)((groups + 15) / 16)), dim3(256), 0, stream, x, ldx, y, ldy,
+                       groups, (int)(K / 256));
+    return hipGetLastError();
+}
+
 size_t quant_rotate_lds_bytes(int64_t K) { return ((size_t)(K / 256) * QR_GSTRIDE + 16) * sizeof(float); }
 
 }  // namespace phi_dev
