@@ -24,6 +24,7 @@
 // lane group g (16 lanes) multiplies columns 32 g .. +31 as two fragments
 // (the sum over k may take them in any order, if A and B agree): packed 4-bit
 // weights are the same 32 columns in one 16-byte read, expanded in registers.
+#include <atomic>
 #include <cmath>
 
 #include "device_common.hpp"
@@ -356,10 +357,18 @@ static hipError_t launch_one(hipStream_t stream, const GemmParams& p) {
     const int64_t blocks = (int64_t)((p.M + 16 * MT - 1) / (16 * MT)) * ((p.N + 16 * NT - 1) / (16 * NT));
     if (blocks > INT32_MAX) return hipErrorInvalidValue;
     constexpr int lds = NW * skinny_region<MT, NT, S, SB>;
-    if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute((const void*)i8_gemm_skinny_kernel<MT, NT, NW, S, SB>,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return e;
+    if (lds > 65536) {  // one attribute call per instantiation and device
+        static std::atomic<uint64_t> set{0};
+        int dev = 0;
+        const hipError_t d = hipGetDevice(&dev);
+        if (d != hipSuccess) return d;
+        const uint64_t bit = dev < 64 ? 1ull << dev : 0;
+        if (!(set.load(std::memory_order_relaxed) & bit)) {
+            const hipError_t e = hipFuncSetAttribute((const void*)i8_gemm_skinny_kernel<MT, NT, NW, S, SB>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            if (e != hipSuccess) return e;
+            set.fetch_or(bit, std::memory_order_relaxed);
+        }
     }
     hipLaunchKernelGGL((i8_gemm_skinny_kernel<MT, NT, NW, S, SB>), dim3((unsigned)blocks), dim3(NW * 64), lds, stream, p);
     return hipGetLastError();
