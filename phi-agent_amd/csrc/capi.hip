@@ -567,6 +567,53 @@ phi_status phi_hip_i8_gemm_residual(phi_stream_t stream, const int8_t* A, int64_
     return check_hip(launch_persist_plan((hipStream_t)stream, p, gk, false, PHI_F32, ldh), who);
 }
 
+// The linear of a few rows as one launch, where it applies (row_linear_ok, no
+// kernel forced by an A/B switch, no tuning-table entry; PHI_ROW_LINEAR=0
+// keeps it out).  Every argument the two-launch form checks is checked first.
+// done: whether the call was made (or refused).
+static phi_status row_linear(const char* who, phi_stream_t stream, const void* x, int x_dtype, int64_t ldx, int64_t M,
+                             int64_t K, const int8_t* W, int64_t ldw, int kt, const float* sW, int sw_scalar,
+                             const void* bias, int bias_dtype, int64_t N, void* C, int c_dtype, int64_t ldc, int8_t* q8,
+                             float* s8, int round_mode, bool* done) {
+    *done = false;
+    if (M > 8 || K > 16384 || N > 16384) return PHI_OK;
+    if (getenv("PHI_GEMM_KERNEL") || getenv("PHI_GEMM_PIPE") || getenv("PHI_GEMM_MIXED") || getenv("PHI_GEMM_T272") ||
+        getenv("PHI_GEMM_SKINNY") || getenv("PHI_QR_ROUNDS") || !phi_dev::env_switch("PHI_ROW_LINEAR", 1, 0, 1))
+        return PHI_OK;
+    phi_gemm_plan plan{};
+    if (tuned_plan(M, N, K, kt, &plan) && plan_is_set(plan)) return PHI_OK;
+    phi_status st;
+    const int bk = bias_kind_of(bias, bias_dtype, &st);
+    if (st != PHI_OK || (bias && !aligned(bias, bk == phi_dev::BIAS_BF16 ? 2 : 4))) return PHI_OK;  // refused below
+    const phi_dev::QrPre pre{};
+    *done = true;
+    st = quant_rotate_check(who, x, x_dtype, M, K, ldx, pre, q8, K, s8, 127.0f, round_mode);
+    if (st != PHI_OK) return st;
+    phi_dev::GemmParams p{};
+    p.B = W;
+    p.sB = sW;
+    p.bias = bias;
+    p.C = C;
+    p.lda = K;
+    p.ldb = ldw;
+    p.ldc = ldc;
+    p.M = (int)M;
+    p.N = (int)N;
+    p.K = (int)K;
+    p.sb_scalar = sw_scalar ? 1 : 0;
+    p.bias_kind = bk;
+    p.c_kind = c_kind_of(c_dtype);
+    p.kt = kt;
+    set_vec_flags(p, c_dtype, ldc);
+    if (!phi_dev::row_linear_ok(p)) {
+        *done = false;
+        return PHI_OK;
+    }
+    return check_hip(phi_dev::launch_row_linear((hipStream_t)stream, p, x, x_dtype == PHI_BF16, ldx,
+                                                round_mode == PHI_ROUND_HALF_EVEN, q8, s8),
+                     who);
+}
+
 phi_status phi_hip_q8_linear(phi_stream_t stream, const void* x, int x_dtype, int64_t ldx,
                              int64_t M, int64_t K, const int8_t* W, int64_t ldw, const float* sW,
                              int sw_scalar, const void* bias, int bias_dtype, int64_t N, void* C,
@@ -578,6 +625,10 @@ phi_status phi_hip_q8_linear(phi_stream_t stream, const void* x, int x_dtype, in
     if (M <= 0) return fail(PHI_ERR_SHAPE, "%s: empty problem", who);
     phi_status st = check_gemm(who, q8, K, W, ldw, M, N, K, s8, sW, C, c_dtype, ldc, false);
     if (st != PHI_OK) return st;
+    bool done;
+    st = row_linear("quant_rotate", stream, x, x_dtype, ldx, M, K, W, ldw, 0, sW, sw_scalar, bias, bias_dtype, N, C, c_dtype,
+                    ldc, q8, s8, round_mode, &done);
+    if (done) return st;
     st = phi_hip_quant_rotate(stream, x, x_dtype, M, K, ldx, q8, K, s8, 127.0f, round_mode, 1);
     if (st != PHI_OK) return st;
     return phi_hip_i8_gemm(stream, q8, K, W, ldw, s8, sW, sw_scalar, bias, bias_dtype, C, c_dtype, ldc, M, N, K,
@@ -780,6 +831,10 @@ phi_status phi_hip_q8_linear_kt(phi_stream_t stream, const void* x, int x_dtype,
     if (K > 16384) return fail(PHI_ERR_UNSUPPORTED, "%s: K=%lld exceeds 16384 (K-tiled activations)", who, (long long)K);
     if (!persist_ok(C, c_dtype, N, K, K, K, ldc))
         return fail(PHI_ERR_UNSUPPORTED, "%s: needs whole 16-byte output pieces on 16-byte aligned C rows", who);
+    bool done;
+    st = row_linear("quant_convrot_kt", stream, x, x_dtype, ldx, M, K, W, K, 1, sW, sw_scalar, bias, bias_dtype, N, C, c_dtype,
+                    ldc, q8, s8, round_mode, &done);
+    if (done) return st;
     st = phi_hip_quant_rotate_kt(stream, x, x_dtype, M, K, ldx, q8, s8, 127.0f, round_mode);
     if (st != PHI_OK) return st;
     return i8_gemm_kt_impl(who, stream, q8, W, s8, sW, sw_scalar, bias, bias_dtype, C, c_dtype, ldc, M, N, K);

@@ -97,6 +97,13 @@ bool skinny_ok(const GemmParams& p, bool w4);
 int skinny_configs();
 int skinny_best(const GemmParams& p, bool w4, int num_cus, double* us);
 hipError_t launch_i8_gemm_skinny(hipStream_t stream, const GemmParams& p, bool w4, int cfg);
+// The linear of a few rows in one launch (row_linear.hip): x rotated and
+// quantised (qmax 127) in every block, q8 (row-major, or K-tiled with p.kt) and
+// s8 written by one.  p.A and p.sA are not read.  row_linear_ok: at most
+// 8 rows and 8192 elements of x (one row: 16384), K % 256 == 0, N <= 16384, skinny_ok.
+bool row_linear_ok(const GemmParams& p);
+hipError_t launch_row_linear(hipStream_t stream, const GemmParams& p, const void* x, bool bf16_in, int64_t ldx,
+                             int half_even, int8_t* q8, float* s8);
 // The same tiles with B as W4 codes (p.B [N, ldb], p.lut, p.group_shift)
 // expanded in LDS; K-tiled A, K % 1024 == 0 (t272w4_ok).
 bool t272w4_ok(const GemmParams& p);

@@ -97,3 +97,40 @@ def test_table_entry_keeps_the_persistent_kernel_and_its_bits(dev):
             assert torch.equal(Q.i8_gemm(A, B, None, None, out_dtype=torch.int32), want)
     finally:
         Q.gemm_plan_clear()
+
+
+@pytest.mark.parametrize("rm", [Q.ROUND_HALF_AWAY, Q.ROUND_HALF_EVEN])
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,K,N", [(1, 256, 8), (1, 3072, 3072), (1, 12288, 96), (1, 16384, 40), (1, 5120, 4104), (2, 4096, 8200),
+                                   (8, 1024, 136), (2, 3072, 1000), (7, 512, 16384), (3, 2048, 64)])
+def test_few_rows_in_one_launch(dev, monkeypatch, xdt, rm, M, K, N):
+    """The one-launch linear against rotate + quantise then GEMM: codes, scales
+    and outputs, with rows that hold an inf, a NaN, huge and tiny values."""
+    x = synth.activations(M, K, seed=M + K).to(xdt)
+    if M > 2:
+        x[1, 5], x[2, 7] = float("inf"), float("nan")
+    if M > 4:
+        x[3] *= 1e-37
+        x[4, :9] = 3e38
+    x = x.to(dev)
+    W, b = synth.int8_weight(N, K, seed=N).to(dev), synth.bias(N, seed=3).to(dev)
+    sW = torch.rand(N, device=dev) * 0.01
+    Wk = Q.pack_k_tiled(W)
+
+    def f(kt, out, bias):
+        q8, s8 = torch.zeros((M * K,), dtype=torch.int8, device=dev), torch.zeros((M,), device=dev)
+        kw = dict(out_dtype=out, s8=s8, round_mode=rm)
+        y = Q.q8_linear_kt(x, Wk, N, sW, bias, q8=q8, **kw) if kt else Q.q8_linear(x, W, sW, bias, q8=q8.view(M, K), **kw)
+        return y, q8, s8
+
+    for kt in (False, True):
+        for out, bias in ((torch.bfloat16, b), (torch.float32, None)):
+            monkeypatch.setenv("PHI_ROW_LINEAR", "0")
+            want = f(kt, out, bias)
+            monkeypatch.delenv("PHI_ROW_LINEAR")
+            got = f(kt, out, bias)
+            torch.cuda.synchronize()
+            for g, w in zip(got, want):
+                v = {2: torch.int16, 4: torch.int32, 1: torch.int8}[g.element_size()]
+                same = (g.view(v) == w.view(v)) | (torch.isnan(g.float()) & torch.isnan(w.float()))
+                assert bool(same.all())
