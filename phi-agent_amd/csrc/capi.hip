@@ -309,6 +309,23 @@ int skinny_choice(const phi_dev::GemmParams& p, bool w4, int G, double other_us)
     return 1.15 * us + 0.5 < other_us ? cfg : -1;
 }
 
+// Whether a problem the persistent kernel refuses only for its output (pieces
+// or rows that are no whole 16 bytes) runs on the pipeline with the
+// element-wise epilogue.  PHI_GEMM_LOOSE=0 keeps it out.
+bool loose_ok(const phi_dev::GemmParams& p, bool pok, bool staged_ok) {
+    const int64_t lim = (int64_t)1 << 23;
+    return !pok && staged_ok && p.K % 256 == 0 && p.lda < lim && p.ldb < lim && p.ldc < lim / 4 && !getenv("PHI_GEMM_KERNEL") &&
+           phi_dev::env_switch("PHI_GEMM_LOOSE", 1, 0, 1);
+}
+
+// The same as persist_us for it: its stores cost a round about 10 us.  Against
+// the register-staged tiles: 4096 x 4101 x 3072 in bf16 139 -> 94 us, 8000 x
+// 11645 x 1024 in fp32 384 -> 261, 2000 x 1001 x 2048 26 -> 17 (whole pieces
+// take 58, 200 and 9).
+double loose_us(const phi_dev::GemmParams& p, int G) {
+    return persist_us(p, false, G) + 3.0 + 10.0 * square_plan_cost(p.M, p.N, G);
+}
+
 // Whether a tuning-table entry says how the persistent kernel runs (and not
 // only the library's own choice, which may be the small-problem kernel).
 bool plan_is_set(const phi_gemm_plan& q) { return q.big_rows >= 0 || q.group_m > 0 || q.split || q.tile != PHI_PLAN_TILE_AUTO; }
@@ -509,8 +526,22 @@ phi_status phi_hip_i8_gemm(phi_stream_t stream, const int8_t* A, int64_t lda, co
     set_vec_flags(p, c_dtype, ldc);
     const bool pok = persist_ok(C, c_dtype, N, K, lda, ldb, ldc);
     if (staged_ok && !pok) {
-        const int cfg = skinny_choice(p, false, num_cus(), tile_us(p, num_cus()));
+        const int G = num_cus();
+        const int cfg = skinny_choice(p, false, G, loose_ok(p, pok, staged_ok) ? loose_us(p, G) : tile_us(p, G));
         if (cfg >= 0) return check_hip(phi_dev::launch_i8_gemm_skinny((hipStream_t)stream, p, false, cfg), who);
+    }
+    if (loose_ok(p, pok, staged_ok)) {
+        const int G = num_cus();
+        const int64_t rows = big_tile_rows(M, N, G);
+        p.loose_bias = p.bias_kind;
+        p.bias_kind = phi_dev::BIAS_NONE;
+        phi_dev::GemmParams big = p, small = p;
+        big.M = (int)rows;
+        small.M = (int)(M - rows);
+        small.A = p.A + rows * lda;
+        if (small.sA) small.sA = p.sA + rows;
+        small.C = (int8_t*)C + rows * ldc * (int64_t)c_elem_bytes(c_dtype);
+        return check_hip(phi_dev::launch_i8_gemm_pipe_loose((hipStream_t)stream, big, small, G), who);
     }
     if (!staged_ok || (ek && strcmp(ek, "any") == 0))
         return check_hip(phi_dev::launch_i8_gemm_any((hipStream_t)stream, p, gemm_cfg_for(M, N)), who);

@@ -45,6 +45,9 @@ struct GemmParams {
     // (w4_banded_bytes, the codes region then the tables region) instead of
     // the checkpoint's code rows and the [N, K / group, 16] table.
     int w4_banded;
+    // The pipeline's element-wise epilogue (epilogue_loose): the bias kind,
+    // while bias_kind is BIAS_NONE.
+    int loose_bias;
 };
 
 // The K-tiled operand layout: rows in strips of 256 (the last strip may be
@@ -81,6 +84,10 @@ hipError_t launch_i8_gemm_persist_mixed(hipStream_t stream, const GemmParams& pb
 // (i8_gemm_pipe.hip).
 hipError_t launch_i8_gemm_pipe(hipStream_t stream, const GemmParams& p, int num_cus, int wave_tile);
 hipError_t launch_i8_gemm_pipe_mixed(hipStream_t stream, const GemmParams& pb, const GemmParams& ps, int num_cus);
+// Both for any N and any pitch and alignment of C's elements (row-major
+// operands, no gate; p.loose_bias in p.bias_kind's place): ps with no rows for
+// one tile size, or pb.
+hipError_t launch_i8_gemm_pipe_loose(hipStream_t stream, const GemmParams& pb, const GemmParams& ps, int num_cus);
 // Persistent kernel on 272 x 192 tiles (i8_gemm_t272.hip): K-tiled operands,
 // row-major ones at 16-byte pitches and addresses, or (b_rm) A K-tiled and B
 // row-major; K % 512 == 0, a gate only with fp32 output, rows x pitch below

@@ -342,7 +342,10 @@ __device__ __forceinline__ NextTile next_tile(const Shape& s, const GemmParams& 
 // la and four B stages at lb (STG bytes each), the epilogue-operand areas
 // eall and the epilogue staging cbuf.  K % 256 == 0.  Returns at once when
 // the workgroup has no tile.
-template <int WT, bool G, bool KT, bool F>
+// L: the element-wise epilogue (epilogue_loose); its stores are more than the
+// NSTORE a tile's first waits leave in flight, which only makes those waits
+// stricter.
+template <int WT, bool G, bool KT, bool F, bool L = false>
 __device__ __forceinline__ void pipe_tiles(const GemmParams& p, int8_t* la, int8_t* lb, int8_t* eall, int8_t* cbuf) {
     using C = PCfg<WT>;
     constexpr int NB = C::NB, DL = C::DL, BM = C::BM;
@@ -489,7 +492,8 @@ __device__ __forceinline__ void pipe_tiles(const GemmParams& p, int8_t* la, int8
                 pstep<WT, 3, false, VWN, false, false, G, KT>(f0, acc, w, p, nt, ln);
             }
             PHI_PIPE_STAMP(WT == 128 ? 0 : 1, i, 1);
-            epilogue<WT, G>(acc, p, cur.m0, cur.n0, w, le);
+            if constexpr (L) epilogue_loose<WT>(acc, p, cur.m0, cur.n0, w, le);
+            else epilogue<WT, G>(acc, p, cur.m0, cur.n0, w, le);
             PHI_PIPE_STAMP(WT == 128 ? 0 : 1, i, 2);
             if (++i == ntile) break;
             cur = nt;
@@ -526,6 +530,17 @@ __global__ __launch_bounds__(256) void i8_gemm_pipe_mixed_kernel(GemmParams pb, 
     PHI_PIPE_STAMP(2, 0, 0);
     pipe_tiles<64, G, KT, F>(ps, la, lb, eall, cbuf);
     PHI_PIPE_TRACE_END
+}
+
+// The same with the element-wise epilogue; either size may have no rows.
+__global__ __launch_bounds__(256) void i8_gemm_pipe_loose_kernel(GemmParams pb, GemmParams ps) {
+    constexpr int STG = PCfg<128>::STG;
+    __shared__ __align__(16) int8_t la[NSTG * STG], lb[NSTG * STG];
+    __shared__ __align__(16) int8_t eall[2 * EBYTES];
+    __shared__ __align__(16) int8_t cbuf[4 * CHUNK];
+    if (pb.M > 0) pipe_tiles<128, false, false, false, true>(pb, la, lb, eall, cbuf);
+    __syncthreads();  // every wave is done with the big tiles' LDS
+    if (ps.M > 0) pipe_tiles<64, false, false, false, true>(ps, la, lb, eall, cbuf);
 }
 
 }  // namespace
@@ -571,6 +586,14 @@ hipError_t launch_i8_gemm_pipe_mixed(hipStream_t stream, const GemmParams& pb, c
         else hipLaunchKernelGGL((i8_gemm_pipe_mixed_kernel<false, false, true>), g3, b3, 0, stream, pb, ps);
     } else if (pb.kt) hipLaunchKernelGGL((i8_gemm_pipe_mixed_kernel<false, true, false>), g3, b3, 0, stream, pb, ps);
     else hipLaunchKernelGGL((i8_gemm_pipe_mixed_kernel<false, false, false>), g3, b3, 0, stream, pb, ps);
+    return hipGetLastError();
+}
+
+hipError_t launch_i8_gemm_pipe_loose(hipStream_t stream, const GemmParams& pb, const GemmParams& ps, int num_cus) {
+    if (pb.K != ps.K || pb.K % (NSTG * PK) != 0 || pb.K < NSTG * PK || pb.kt || pb.gate) return hipErrorInvalidValue;
+    const int big = ((pb.M + 255) / 256) * ((pb.N + 255) / 256), small = ((ps.M + 127) / 128) * ((ps.N + 127) / 128);
+    const int most = big > small ? big : small;
+    hipLaunchKernelGGL(i8_gemm_pipe_loose_kernel, dim3(most < num_cus ? most : num_cus), dim3(256), 0, stream, pb, ps);
     return hipGetLastError();
 }
 

@@ -226,7 +226,8 @@ struct SkinnyCfg {
     int mt, nt, nw, s;
 };
 constexpr SkinnyCfg kSkinny[] = {{1, 1, 8, 2}, {1, 2, 8, 1}, {1, 4, 8, 1}, {2, 1, 8, 1}, {2, 2, 8, 1}, {2, 4, 8, 1},
-                                 {4, 1, 8, 1}, {4, 2, 8, 1}, {4, 4, 8, 1}, {5, 2, 8, 1}, {5, 4, 8, 1}, {6, 4, 4, 2}};
+                                 {4, 1, 8, 1}, {4, 2, 8, 1}, {4, 4, 8, 1}, {5, 2, 8, 1}, {5, 4, 8, 1}, {6, 4, 4, 2},
+                                 {3, 8, 4, 1}, {5, 8, 4, 1}};
 constexpr int kSkinnyCfgs = (int)(sizeof kSkinny / sizeof kSkinny[0]);
 
 int skinny_configs() { return kSkinnyCfgs; }
@@ -255,7 +256,8 @@ int skinny_best(const GemmParams& p, bool w4, int num_cus, double* us) {
         const double ti = skinny_us(p, w4, num_cus, i);
         if (ti < t) t = ti, best = i;
     }
-    *us = t;
+    // Element-wise stores (odd columns or pitch): 4.5 us a million outputs.
+    *us = t + (p.c_vec && p.N % 4 == 0 ? 0.0 : 4.5e-6 * p.M * p.N);
     return best;
 }
 
@@ -289,10 +291,13 @@ static hipError_t launch_one(hipStream_t stream, const GemmParams& p) {
 
 template <int MT, int NT, int NW, int S>
 static hipError_t launch_cfg(hipStream_t stream, const GemmParams& p, int sb) {
+    // A second stage where the partial sums' region holds one anyway.
+    constexpr int SL = S == 1 && 2 * skinny_stage<MT, NT, SB_LUT> <= MT * NT * 1024 ? 2 : S;
+    constexpr int S4 = S == 1 && 2 * skinny_stage<MT, NT, SB_S4> <= MT * NT * 1024 ? 2 : S;
     switch (sb) {
         case SB_I8: return launch_one<MT, NT, NW, S, SB_I8>(stream, p);
-        case SB_LUT: return launch_one<MT, NT, NW, S, SB_LUT>(stream, p);
-        default: return launch_one<MT, NT, NW, S, SB_S4>(stream, p);
+        case SB_LUT: return launch_one<MT, NT, NW, SL, SB_LUT>(stream, p);
+        default: return launch_one<MT, NT, NW, S4, SB_S4>(stream, p);
     }
 }
 
@@ -315,7 +320,9 @@ hipError_t launch_i8_gemm_skinny(hipStream_t stream, const GemmParams& p, bool w
         case 8: return launch_at<8>(stream, p, sb);
         case 9: return launch_at<9>(stream, p, sb);
         case 10: return launch_at<10>(stream, p, sb);
-        default: return launch_at<11>(stream, p, sb);
+        case 11: return launch_at<11>(stream, p, sb);
+        case 12: return launch_at<12>(stream, p, sb);
+        default: return launch_at<13>(stream, p, sb);
     }
 }
 

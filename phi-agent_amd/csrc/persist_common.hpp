@@ -352,5 +352,72 @@ __device__ __forceinline__ void epilogue(v16i (&acc)[WT / 32][WT / 32], const Ge
     }
 }
 
+// The epilogue for output rows that hold no whole 16-byte pieces (any N, any
+// pitch and alignment of C's elements): the same values through the same
+// staging in fp32, read back one element a lane and stored a
+// piece of 32 columns of two rows at a time.  Cached stores: neighbouring
+// pieces meet in L2 before they leave it (8000 x 11645 in fp32, non-temporal
+// 349 us, cached 261).  The bias is
+// read from memory (its staged copy comes in pairs of bf16, and N may be odd);
+// its kind is in loose_bias, bias_kind is BIAS_NONE.
+template <int WT>
+__device__ __forceinline__ void epilogue_loose(v16i (&acc)[WT / 32][WT / 32], const GemmParams& p, int m0, int n0,
+                                               const EpiWave& w, const int8_t* e) {
+    constexpr int NB = WT / 32;
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+#pragma unroll
+        for (int i = 0; i < NB; i++) asm volatile("" : "+a"(acc[j][i]));
+    int8_t* lc = w.lc;
+    const int colw = n0 + w.wn * WT, roww = m0 + w.wm * WT;
+    float sa[NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++) sa[i] = *(const float*)(e + (w.wm * WT + i * 32 + w.lrow) * 4);
+#pragma unroll
+    for (int c0 = 0; c0 < WT; c0 += 64) {
+        const int n = min(colw + c0 + w.lane, p.N - 1);
+        float b = 0.0f;
+        if (p.loose_bias == BIAS_F32) b = ((const float*)p.bias)[n];
+        else if (p.loose_bias == BIAS_BF16) b = bf16_to_f32(((const uint16_t*)p.bias)[n]);
+        *(float*)(lc + 4096 + (c0 + w.lane) * 4) = b;
+    }
+    const bool bf = p.c_kind == C_BF16;
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        v4f sb[4], bz[4];
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            col_operands(w, e, w.wn * WT + j * 32 + 8 * g + 4 * w.lhalf, j * 32 + 8 * g + 4 * w.lhalf, sb[g], bz[g]);
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            v16i blk = acc[j][i];
+            asm volatile("" : "+v"(blk));
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                u32x4 o;
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    o[q] = p.c_kind == C_I32 ? (unsigned)blk[4 * g + q]
+                                             : __float_as_uint(fmaf((float)blk[4 * g + q] * sa[i], sb[g][q], bz[g][q]));
+                const int slot = (2 * g + w.lhalf) ^ ((w.lrow >> 1) & 7);
+                *(u32x4*)(lc + w.lrow * 128 + slot * 16) = o;
+            }
+            // A wave's LDS accesses complete in order: these reads see its writes.
+            const int c = w.lane & 31, col = colw + j * 32 + c, row0 = roww + i * 32 + w.lhalf;
+            const int64_t off = (int64_t)row0 * p.ldc + col;
+            const int live = col < p.N ? p.M - row0 : 0;
+#pragma unroll 4
+            for (int t = 0; t < 32; t += 2) {
+                const int r = t + w.lhalf;
+                const uint32_t v = *(const uint32_t*)(lc + r * 128 + (((c >> 2) ^ ((r >> 1) & 7)) * 16) + (c & 3) * 4);
+                if (t >= live) continue;
+                if (bf) ((uint16_t*)p.C)[off + t * p.ldc] = (uint16_t)f32_to_bf16(__uint_as_float(v));
+                else ((uint32_t*)p.C)[off + t * p.ldc] = v;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
 }  // namespace persist
 }  // namespace phi_dev

@@ -181,15 +181,16 @@ __global__ __launch_bounds__(256) void lora_fold_kernel(float* w, int64_t ldw, i
     }
 }
 
-// The same for 16 rows x 256 columns a wave, four columns a lane, four ranks
-// at a time: A's rows are read once for 16 weight rows; lane 4 i + j holds
+// The same for 8 rows x 256 columns a wave, four columns a lane, four ranks at
+// a time: A's rows are read once for 8 weight rows; lane 4 i + j (< 32) holds
 // rank j of row i of the scaled B entries, handed to the wave as scalars
 // (v_readlane), with the entries to skip (zeros, ranks past the last) as one
 // 64-bit mask.  The two roundings an entry bind it: 8 VALU instructions and
 // the readlane for 4 columns, 66 us of the whole chip at 12288 x 3072, rank 32,
-// beside 302 MB read and written: 99 us, the general kernel 636.  k % 4 == 0, w
+// beside 302 MB read and written: 87 us (16
+// rows a wave 96, at half the waves a SIMD), the general kernel 636.  k % 4 == 0, w
 // and A rows 16-byte aligned.
-constexpr int LF_ROWS = 16;
+constexpr int LF_ROWS = 8;
 __global__ __launch_bounds__(256) void lora_fold_tile_kernel(float* __restrict__ w, int64_t ldw, int64_t rows, int64_t k,
                                                              const float* __restrict__ A, const float* __restrict__ B,
                                                              int64_t rank, float scale, int col_blocks) {
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(256) void lora_fold_tile_kernel(float* __restrict__
     // Columns past the last repeat them (their lanes take part in the
     // readlanes) and are not stored.
     const int64_t cw = (int64_t)(blockIdx.x % col_blocks) * 256 + lane * 4, c = min(cw, k - 4);
-    const float* brow = B + min(o0 + (lane >> 2), rows - 1) * rank;
+    const float* brow = B + min(o0 + (lane >> 2) % LF_ROWS, rows - 1) * rank;
     float4 acc[LF_ROWS], a[4], an[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) an[j] = *(const float4*)(A + min((int64_t)j, rank - 1) * k + c);

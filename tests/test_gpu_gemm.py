@@ -318,3 +318,24 @@ def test_tile_size_plan_epilogue(dev, orc, monkeypatch, out):
     want = orc.epilogue(acc, sa.numpy(), sb.numpy(), u16(bias), out=out)
     got = u16(C) if out == "bf16" else C.cpu().numpy().view(np.uint32)
     assert np.array_equal(got, want if out == "bf16" else want.view(np.uint32))
+
+
+@pytest.mark.parametrize("out", [torch.int32, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,pad", [(1, 1, 256, 0), (129, 131, 512, 1), (300, 259, 768, 0), (513, 1021, 256, 3), (2000, 1001, 1024, 2)])
+def test_odd_columns_on_the_pipeline(dev, monkeypatch, out, M, N, K, pad):
+    """Outputs that hold no whole 16-byte pieces: the pipeline's element-wise
+    epilogue against the register-staged tiles, padding columns untouched, C
+    one element off any wider alignment, a bias whose columns are odd."""
+    monkeypatch.setenv("PHI_GEMM_SKINNY", "off")
+    A, B = synth.int8_weight(M, K, seed=M).to(dev), synth.int8_weight(N, K, seed=N + 1).to(dev)
+    sA, sB = torch.rand(M, device=dev), torch.rand(N, device=dev)
+    for bias in (None, torch.randn(N, device=dev), torch.randn(N, device=dev).bfloat16()):
+        got = []
+        for loose in ("0", "1"):
+            monkeypatch.setenv("PHI_GEMM_LOOSE", loose)
+            buf = torch.zeros(M * (N + pad) + 1, dtype=out, device=dev)
+            C = buf[1:].view(M, N + pad)[:, :N]
+            Q.i8_gemm(A, B, sA, sB, bias, C=C)
+            torch.cuda.synchronize()
+            got.append(buf)
+        assert torch.equal(got[0], got[1])
