@@ -311,9 +311,14 @@ int skinny_choice(const phi_dev::GemmParams& p, bool w4, int G, double other_us)
 
 // Whether a problem the persistent kernel refuses only for its output (pieces
 // or rows that are no whole 16 bytes) runs on the pipeline with the
-// element-wise epilogue.  PHI_GEMM_LOOSE=0 keeps it out.
+// element-wise epilogue.  Between one and two rounds of 128 x 128 tiles the
+// register-staged kernel keeps it: two of its blocks share a CU, and the two
+// take the same time (1023 x 4101 x 3072: 41 us each; 1358 x 4391 x 2048: 33
+// against 34).  PHI_GEMM_LOOSE=0 keeps the pipeline out, 1 takes both.
 bool loose_ok(const phi_dev::GemmParams& p, bool pok, bool staged_ok) {
     const int64_t lim = (int64_t)1 << 23;
+    const int64_t big = ((int64_t)p.M + 255) / 256 * ((p.N + 255) / 256), small = ((int64_t)p.M + 127) / 128 * ((p.N + 127) / 128);
+    if (big < 128 && small > num_cus() && !phi_dev::env_switch("PHI_GEMM_LOOSE", 0, 0, 1)) return false;
     return !pok && staged_ok && p.K % 256 == 0 && p.lda < lim && p.ldb < lim && p.ldc < lim / 4 && !getenv("PHI_GEMM_KERNEL") &&
            phi_dev::env_switch("PHI_GEMM_LOOSE", 1, 0, 1);
 }
