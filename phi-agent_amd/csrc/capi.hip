@@ -621,6 +621,11 @@ static phi_status row_linear(const char* who, phi_stream_t stream, const void* x
     phi_status st;
     const int bk = bias_kind_of(bias, bias_dtype, &st);
     if (st != PHI_OK || (bias && !aligned(bias, bk == phi_dev::BIAS_BF16 ? 2 : 4))) return PHI_OK;  // refused below
+    // Every block reads all of x, some after others have stored: an output or
+    // scratch that shares memory with x (a linear in place) takes two launches.
+    const uintptr_t xb = (uintptr_t)x, xe = xb + (uintptr_t)(((M - 1) * ldx + K) * (x_dtype == PHI_BF16 ? 2 : 4));
+    auto meets = [&](const void* b, int64_t bytes) { return (uintptr_t)b < xe && xb < (uintptr_t)b + (uintptr_t)bytes; };
+    if (ldx < K || meets(C, ((M - 1) * ldc + N) * (int64_t)c_elem_bytes(c_dtype)) || meets(q8, M * K) || meets(s8, M * 4)) return PHI_OK;
     const phi_dev::QrPre pre{};
     *done = true;
     st = quant_rotate_check(who, x, x_dtype, M, K, ldx, pre, q8, K, s8, 127.0f, round_mode);

@@ -134,3 +134,17 @@ def test_few_rows_in_one_launch(dev, monkeypatch, xdt, rm, M, K, N):
                 v = {2: torch.int16, 4: torch.int32, 1: torch.int8}[g.element_size()]
                 same = (g.view(v) == w.view(v)) | (torch.isnan(g.float()) & torch.isnan(w.float()))
                 assert bool(same.all())
+
+
+@pytest.mark.parametrize("K", [256, 3072])
+def test_few_rows_in_place(dev, monkeypatch, K):
+    """An output over the input takes two launches: all of x is read before the first store."""
+    W, sW = synth.int8_weight(K, K, seed=2).to(dev), torch.rand(K, device=dev) * 0.01
+    x = synth.activations(1, K, seed=1).to(dev)
+    q8, s8 = torch.empty((1, K), dtype=torch.int8, device=dev), torch.empty((1,), device=dev)
+    want = Q.q8_linear(x, W, sW, q8=q8, s8=s8)
+    for _ in range(8):
+        y = x.clone()
+        Q.q8_linear(y, W, sW, q8=q8, s8=s8, C=y)
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
