@@ -343,7 +343,8 @@ phi_status phi_hip_w4a8_prepare(phi_stream_t stream, const phi_w4a8_weight* w, i
  *     The expand-once path and the LDS path (K <= 16384) keep the activation
  *     codes in the K-tiled layout (phi_hip_pack_k_tiled), so q8 then holds
  *     them K-tiled; s8 is the same on every path.  A problem too small for
- *     either expands in registers, its codes read once, q8 row-major.
+ *     either expands in registers, its codes read once, q8 in the layout
+ *     that the path above would leave.
  */
 phi_status phi_hip_w4a8_linear(phi_stream_t stream, const void* x, int x_dtype, int64_t ldx,
                                int64_t M, int64_t K, const uint8_t* codes,

@@ -295,7 +295,7 @@ double w4a8_us(const phi_dev::GemmParams& p, int G, bool workspace) {
 
 // The small-problem kernel's tile for p where the model says it beats
 // `other_us`, or -1.  A kernel forced by an A/B switch keeps its problems;
-// PHI_GEMM_SKINNY=0..11 forces a tile of this one, any other value turns it
+// PHI_GEMM_SKINNY=0..13 forces a tile of this one, any other value turns it
 // off.
 int skinny_choice(const phi_dev::GemmParams& p, bool w4, int G, double other_us) {
     if (!phi_dev::skinny_ok(p, w4)) return -1;
@@ -1030,68 +1030,6 @@ phi_status phi_hip_w4a8_linear(phi_stream_t stream, const void* x, int x_dtype, 
     // without a workspace it is the in-register path wherever it applies.
     // A kernel forced by PHI_GEMM_KERNEL keeps its own path.
     const int w4t = phi_dev::env_switch("PHI_W4_T272", -1, 0, 1);
-    phi_dev::GemmParams sp{};
-    sp.A = q8;
-    sp.B = (const int8_t*)codes;
-    sp.sA = s8;
-    sp.sB = s_w;
-    sp.bias = bias;
-    sp.C = C;
-    sp.lda = K;
-    sp.ldb = codes_row_bytes;
-    sp.ldc = ldc;
-    sp.M = (int)M;
-    sp.N = (int)N;
-    sp.K = (int)K;
-    sp.bias_kind = bk;
-    sp.c_kind = c_kind_of(c_dtype);
-    sp.lut = lut;
-    sp.lut_groups = K / group;
-    while ((1ll << sp.group_shift) < group) sp.group_shift++;
-    set_vec_flags(sp, c_dtype, ldc);
-    const int skinny = w4t < 0 ? skinny_choice(sp, true, num_cus(), w4a8_us(sp, num_cus(), workspace && need > 0 && ws_bytes >= need)) : -1;
-    if (skinny >= 0) {
-        st = phi_hip_quant_rotate(stream, x, x_dtype, M, K, ldx, q8, K, s8, 127.0f, round_mode, 1);
-        if (st != PHI_OK) return st;
-        return check_hip(phi_dev::launch_i8_gemm_skinny((hipStream_t)stream, sp, true, skinny), who);
-    }
-    if (!e && w4t != 0 && (w4t == 1 || !(need > 0 && workspace && ws_bytes >= need)) && K <= 16384 &&
-        aligned(q8, 16) && aligned(codes, 16) && codes_row_bytes % 16 == 0 &&
-        persist_ok(C, c_dtype, N, K, K, codes_row_bytes, ldc)) {
-        phi_dev::GemmParams q{};
-        q.A = q8;
-        q.B = (const int8_t*)codes;
-        q.sA = s8;
-        q.sB = s_w;
-        q.bias = bias;
-        q.C = C;
-        q.lda = K;
-        q.ldb = codes_row_bytes;
-        q.ldc = ldc;
-        q.M = (int)M;
-        q.N = (int)N;
-        q.K = (int)K;
-        q.sb_scalar = 0;
-        q.bias_kind = bk;
-        q.c_kind = c_kind_of(c_dtype);
-        q.group_m = 4;
-        q.lut = lut;
-        q.lut_groups = K / group;
-        int gs = 0;
-        while ((1ll << gs) < group) gs++;
-        q.group_shift = gs;
-        q.kt = 1;
-        set_vec_flags(q, c_dtype, ldc);
-        if (phi_dev::t272w4_ok(q)) {
-            st = phi_hip_quant_rotate_kt(stream, x, x_dtype, M, K, ldx, q8, s8, 127.0f, round_mode);
-            if (st != PHI_OK) return st;
-            return check_hip(phi_dev::launch_i8_gemm_t272w4((hipStream_t)stream, q, num_cus()), who);
-        }
-    }
-    const bool expand = !force_staged && need > 0 && workspace && ws_bytes >= need && aligned(workspace, 16) &&
-                        aligned(codes, 16) && codes_row_bytes % 16 == 0 && persist_ok(C, c_dtype, N, K, K, K, ldc);
-    const char* ekt = getenv("PHI_GEMM_KT");
-    const bool kt = expand && K <= 16384 && aligned(q8, 16) && !(ekt && ekt[0] == '0');
     phi_dev::GemmParams p{};
     p.A = q8;
     p.B = (const int8_t*)codes;
@@ -1114,6 +1052,33 @@ phi_status phi_hip_w4a8_linear(phi_stream_t stream, const void* x, int x_dtype, 
     int sh = 0;
     while ((1ll << sh) < group) sh++;
     p.group_shift = sh;
+    phi_dev::GemmParams q = p;  // on K-tiled activations
+    q.kt = 1;
+    set_vec_flags(q, c_dtype, ldc);
+    const bool in_lds = !e && w4t != 0 && (w4t == 1 || !(need > 0 && workspace && ws_bytes >= need)) && K <= 16384 &&
+                        aligned(q8, 16) && aligned(codes, 16) && codes_row_bytes % 16 == 0 &&
+                        persist_ok(C, c_dtype, N, K, K, codes_row_bytes, ldc) && phi_dev::t272w4_ok(q);
+    const bool expand = !force_staged && need > 0 && workspace && ws_bytes >= need && aligned(workspace, 16) &&
+                        aligned(codes, 16) && codes_row_bytes % 16 == 0 && persist_ok(C, c_dtype, N, K, K, K, ldc);
+    const char* ekt = getenv("PHI_GEMM_KT");
+    const bool kt = expand && K <= 16384 && aligned(q8, 16) && !(ekt && ekt[0] == '0');
+    // The small-problem kernel, on the activation layout that the path it
+    // stands in for leaves in q8.
+    phi_dev::GemmParams sp = q;
+    sp.kt = in_lds || kt;
+    sp.b_rm = 1;
+    const int skinny = w4t < 0 ? skinny_choice(sp, true, num_cus(), w4a8_us(sp, num_cus(), workspace && need > 0 && ws_bytes >= need)) : -1;
+    if (skinny >= 0) {
+        st = sp.kt ? phi_hip_quant_rotate_kt(stream, x, x_dtype, M, K, ldx, q8, s8, 127.0f, round_mode)
+                   : phi_hip_quant_rotate(stream, x, x_dtype, M, K, ldx, q8, K, s8, 127.0f, round_mode, 1);
+        if (st != PHI_OK) return st;
+        return check_hip(phi_dev::launch_i8_gemm_skinny((hipStream_t)stream, sp, true, skinny), who);
+    }
+    if (in_lds) {
+        st = phi_hip_quant_rotate_kt(stream, x, x_dtype, M, K, ldx, q8, s8, 127.0f, round_mode);
+        if (st != PHI_OK) return st;
+        return check_hip(phi_dev::launch_i8_gemm_t272w4((hipStream_t)stream, q, num_cus()), who);
+    }
     // With K-tiled activations the expansion runs as extra blocks of the
     // prologue's launch, beside the rotation (PHI_W4_FUSE=0: two launches).
     const bool fuse = kt && phi_dev::w4_expand_ok(p, (const int8_t*)workspace, true) &&

@@ -1,7 +1,7 @@
 """The small-problem GEMM (K split over a block's waves) against the other
 kernels: the int32 sums are exact on both and the epilogue is the same, so
 every output is bit-identical.  Its tiles are forced one by one over shapes
-around their edges (PHI_GEMM_SKINNY=0..11; "off" keeps it out)."""
+around their edges (PHI_GEMM_SKINNY=0..13; "off" keeps it out)."""
 import numpy as np
 import pytest
 import torch
@@ -26,7 +26,7 @@ def both(monkeypatch, cfg, f):
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
-@pytest.mark.parametrize("cfg", range(12))
+@pytest.mark.parametrize("cfg", range(14))
 def test_tiles_int8(dev, monkeypatch, cfg, M, N, K):
     g = torch.Generator().manual_seed(M + N + K)
     A, B = synth.int8_weight(M, K, seed=M).to(dev), synth.int8_weight(N, K, seed=N).to(dev)
@@ -59,7 +59,7 @@ def test_tiles_odd_columns_and_pitches(dev, monkeypatch, cfg, out):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 8, 512), (33, 72, 1024), (81, 136, 2560)])
-@pytest.mark.parametrize("cfg", range(12))
+@pytest.mark.parametrize("cfg", range(14))
 def test_tiles_4bit(dev, monkeypatch, cfg, M, N, K):
     g = torch.Generator().manual_seed(K)
     A = synth.int8_weight(M, K, seed=5).to(dev)
@@ -71,7 +71,15 @@ def test_tiles_4bit(dev, monkeypatch, cfg, M, N, K):
     for group in (64, 128, 512):
         codes, s_rel, sch, corr = (t.to(dev) for t in synth.w4a8_weight(N, K, group, seed=7))
         lut, sw = Q.w4a8_prepare(codes, s_rel, Q.F16, sch, k=K, group=group, correction=corr)
-        both(monkeypatch, cfg, lambda: Q.w4a8_linear(x, codes, lut, sw, group=group, out_dtype=torch.float32))
+        q8 = torch.empty((M * K,), dtype=torch.int8, device=dev)
+        for ws in (None, Q.w4a8_workspace(M, N, K, group, dev)):
+
+            def f():
+                """Outputs, and the activation codes in the layout of the path it stands in for."""
+                y = Q.w4a8_linear(x, codes, lut, sw, group=group, out_dtype=torch.float32, q8=q8.view(M, K), workspace=ws)
+                return torch.cat([y.flatten(), q8.float()])
+
+            both(monkeypatch, cfg, f)
 
 
 def test_rule_matches_oracle(dev, orc):
