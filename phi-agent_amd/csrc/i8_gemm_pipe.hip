@@ -342,9 +342,10 @@ __device__ __forceinline__ NextTile next_tile(const Shape& s, const GemmParams& 
 // la and four B stages at lb (STG bytes each), the epilogue-operand areas
 // eall and the epilogue staging cbuf.  K % 256 == 0.  Returns at once when
 // the workgroup has no tile.
-// L: the element-wise epilogue (epilogue_loose); its stores are more than the
-// NSTORE a tile's first waits leave in flight, which only makes those waits
-// stricter.
+// L: the element-wise epilogue (epilogue_loose), which issues any number of
+// stores.  The first two waits of a tile (VWR) count on NSTORE of them after
+// the stages they wait for; with L those stages have landed before the first
+// store (the wait in epilogue_loose), whatever the count.
 template <int WT, bool G, bool KT, bool F, bool L = false>
 __device__ __forceinline__ void pipe_tiles(const GemmParams& p, int8_t* la, int8_t* lb, int8_t* eall, int8_t* cbuf) {
     using C = PCfg<WT>;

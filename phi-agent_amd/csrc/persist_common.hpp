@@ -360,6 +360,11 @@ __device__ __forceinline__ void epilogue(v16i (&acc)[WT / 32][WT / 32], const Ge
 // 349 us, cached 261).  The bias is
 // read from memory (its staged copy comes in pairs of bf16, and N may be odd);
 // its kind is in loose_bias, bias_kind is BIAS_NONE.
+//
+// The stores are branched around past M and N: a wave may issue none.  The
+// next tile's first waits leave as many memory operations in flight as the
+// other epilogues store, so every load the caller has issued (the next tile's
+// stages) is waited for here, before the first store.
 template <int WT>
 __device__ __forceinline__ void epilogue_loose(v16i (&acc)[WT / 32][WT / 32], const GemmParams& p, int m0, int n0,
                                                const EpiWave& w, const int8_t* e) {
@@ -381,6 +386,9 @@ __device__ __forceinline__ void epilogue_loose(v16i (&acc)[WT / 32][WT / 32], co
         else if (p.loose_bias == BIAS_BF16) b = bf16_to_f32(((const uint16_t*)p.bias)[n]);
         *(float*)(lc + 4096 + (c0 + w.lane) * 4) = b;
     }
+    __builtin_amdgcn_sched_barrier(0);
+    wait_all();
+    __builtin_amdgcn_sched_barrier(0);
     const bool bf = p.c_kind == C_BF16;
 #pragma unroll
     for (int j = 0; j < NB; j++) {

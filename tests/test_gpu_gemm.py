@@ -339,3 +339,25 @@ def test_odd_columns_on_the_pipeline(dev, monkeypatch, out, M, N, K, pad):
             torch.cuda.synchronize()
             got.append(buf)
         assert torch.equal(got[0], got[1])
+
+
+# (rows, columns): 255 tiles of 256 x 256 and 66 of 128 x 128 in one launch;
+# the same with a last row tile of one row; several 256 x 256 tiles a
+# workgroup; two 128 x 128 tiles a workgroup, the last of one row.
+@pytest.mark.parametrize("out", [torch.int32, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(4096, 4101, 256), (4096, 4101, 512), (4097, 4101, 512), (8000, 11645, 256), (8000, 11645, 512),
+                                   (1025, 4101, 256), (1025, 4101, 768)])
+def test_odd_columns_over_several_tiles(dev, monkeypatch, out, M, N, K):
+    """The element-wise epilogue between tiles: a wave with nothing to store
+    (all of its columns past N, or its rows past M) goes on to the next tile's
+    stages.  Against the register-staged tiles."""
+    monkeypatch.setenv("PHI_GEMM_SKINNY", "off")
+    A, B = synth.int8_weight(M, K, seed=M, device=dev), synth.int8_weight(N, K, seed=N + 1, device=dev)
+    sA, sB = torch.rand(M, device=dev), torch.rand(N, device=dev)
+    for bias in (None, torch.randn(N, device=dev), torch.randn(N, device=dev).bfloat16()):
+        got = []
+        for loose in ("0", "1"):
+            monkeypatch.setenv("PHI_GEMM_LOOSE", loose)
+            got.append(Q.i8_gemm(A, B, sA, sB, bias, out_dtype=out))
+            torch.cuda.synchronize()
+        assert torch.equal(got[0], got[1])
