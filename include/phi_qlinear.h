@@ -252,9 +252,12 @@ int64_t phi_hip_big_tile_rows(int64_t M, int64_t N);
  * Every plan gives the same bits; only the time differs.  The table is
  * process-wide and thread-safe; the host layer's GemmTuneStore sweeps,
  * persists and loads it.  _set with plan NULL removes the shape's entry;
- * _get returns the plan a launch of that shape runs, the tile shape resolved
- * (tuned = 1 when it comes from the table).  PHI_GEMM_T272=0 / 1 in the
- * environment overrides the tile shape (an A/B switch). */
+ * _get returns the persistent GEMM's plan for the shape, the tile shape
+ * resolved (tuned = 1 when it comes from the table).  A launch runs that plan
+ * unless phi_hip_gemm_is_small says that the small-problem kernel takes the
+ * shape: then it is what would run without that kernel, and handing it to _set
+ * (every field is set) takes the shape away from it.  PHI_GEMM_T272=0 / 1 in
+ * the environment overrides the tile shape (an A/B switch). */
 #define PHI_PLAN_TILE_AUTO 0
 #define PHI_PLAN_TILE_SQUARE 1
 #define PHI_PLAN_TILE_272 2
@@ -267,6 +270,10 @@ typedef struct phi_gemm_plan {
 } phi_gemm_plan;
 phi_status phi_hip_gemm_plan_set(int64_t M, int64_t N, int64_t K, int k_tiled, const phi_gemm_plan* plan);
 phi_status phi_hip_gemm_plan_get(int64_t M, int64_t N, int64_t K, int k_tiled, phi_gemm_plan* plan, int* tuned);
+/* 1 where the small-problem kernel takes launches of the shape (bf16 output,
+ * whole 16-byte rows): the library's model says it is faster and the table has
+ * no entry for the shape that sets a field.  0 elsewhere. */
+int phi_hip_gemm_is_small(int64_t M, int64_t N, int64_t K, int k_tiled);
 int64_t phi_hip_gemm_plan_count(void);
 void phi_hip_gemm_plan_clear(void);
 

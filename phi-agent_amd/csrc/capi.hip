@@ -781,6 +781,25 @@ phi_status phi_hip_gemm_plan_get(int64_t M, int64_t N, int64_t K, int k_tiled, p
     return ok();
 }
 
+int phi_hip_gemm_is_small(int64_t M, int64_t N, int64_t K, int k_tiled) {
+    if (M <= 0 || N <= 0 || K <= 0 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return 0;
+    if (!persist_ok(nullptr, PHI_BF16, N, K, K, K, N)) return 0;
+    phi_gemm_plan plan{};
+    if (tuned_plan(M, N, K, k_tiled, &plan) && plan_is_set(plan)) return 0;
+    phi_dev::GemmParams p{};
+    p.M = (int)M;
+    p.N = (int)N;
+    p.K = (int)K;
+    p.lda = K;
+    p.ldb = K;
+    p.ldc = N;
+    p.c_kind = phi_dev::C_BF16;
+    p.kt = k_tiled ? 1 : 0;
+    set_vec_flags(p, PHI_BF16, N);
+    const int G = num_cus();
+    return skinny_choice(p, false, G, persist_us(p, false, G)) >= 0 ? 1 : 0;
+}
+
 int64_t phi_hip_gemm_plan_count(void) { return g_plan_count.load(std::memory_order_acquire); }
 
 void phi_hip_gemm_plan_clear(void) {

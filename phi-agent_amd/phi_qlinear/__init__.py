@@ -80,7 +80,7 @@ EXPORTS = ["phi_hip_last_error", "phi_hip_abi_version", "phi_hip_quant_rotate", 
            "phi_hip_quant_rotate_kt", "phi_hip_big_tile_rows",
            "phi_hip_quant_rotate_mod_kt", "phi_hip_quant_rotate_act_kt", "phi_hip_i8_gemm_residual_kt",
            "phi_hip_dequant_fp4_rows", "phi_hip_gemm_plan_set", "phi_hip_gemm_plan_get", "phi_hip_gemm_plan_count",
-           "phi_hip_gemm_plan_clear", "phi_hip_w4a8_banded_bytes", "phi_hip_w4a8_pack_banded",
+           "phi_hip_gemm_plan_clear", "phi_hip_gemm_is_small", "phi_hip_w4a8_banded_bytes", "phi_hip_w4a8_pack_banded",
            "phi_hip_w4a8_linear_banded"]
 
 _lib = None
@@ -129,6 +129,7 @@ def load() -> ctypes.CDLL:
     L.phi_hip_dequant_fp4_rows.argtypes = [P, P, I64, I64, I64, I64, P, I64, I64, I64, P, I, P, I64]
     L.phi_hip_gemm_plan_set.argtypes = [I64, I64, I64, I, ctypes.POINTER(GemmPlan)]
     L.phi_hip_gemm_plan_get.argtypes = [I64, I64, I64, I, ctypes.POINTER(GemmPlan), ctypes.POINTER(ctypes.c_int)]
+    L.phi_hip_gemm_is_small.argtypes = [I64, I64, I64, I]
     L.phi_hip_gemm_plan_count.restype = I64
     L.phi_hip_gemm_plan_clear.restype = None
     L.phi_hip_lora_fold.argtypes = [P, P, I64, I64, I64, P, P, I64, F]
@@ -607,12 +608,18 @@ def gemm_plan_set(M: int, N: int, K: int, *, k_tiled: bool = False, big_rows: in
 
 
 def gemm_plan_get(M: int, N: int, K: int, *, k_tiled: bool = False) -> dict:
-    """The plan a GEMM of this shape runs: {big_rows, group_m, split, tile,
-    tuned}, the tile shape resolved (PLAN_TILE_SQUARE or PLAN_TILE_272)."""
+    """The persistent GEMM's plan for this shape: {big_rows, group_m, split,
+    tile, tuned}, the tile shape resolved (PLAN_TILE_SQUARE or PLAN_TILE_272).
+    It is what runs unless gemm_is_small."""
     plan, tuned = GemmPlan(), ctypes.c_int(0)
     _check(load().phi_hip_gemm_plan_get(M, N, K, 1 if k_tiled else 0, ctypes.byref(plan), ctypes.byref(tuned)))
     return {"big_rows": plan.big_rows, "group_m": plan.group_m, "split": bool(plan.split), "tile": plan.tile,
             "tuned": bool(tuned.value)}
+
+
+def gemm_is_small(M: int, N: int, K: int, *, k_tiled: bool = False) -> bool:
+    """Whether the small-problem kernel takes a GEMM of this shape (phi_hip_gemm_is_small)."""
+    return bool(load().phi_hip_gemm_is_small(M, N, K, 1 if k_tiled else 0))
 
 
 def gemm_plan_clear() -> None:

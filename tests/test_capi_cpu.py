@@ -361,3 +361,25 @@ def test_gemm_plan_table(lib):
     assert Q.gemm_plan_count() == 1
     Q.gemm_plan_clear()
     assert Q.gemm_plan_count() == 0
+
+
+def test_gemm_is_small_follows_the_table(lib):
+    """Which shapes the small-problem kernel takes (256 CUs with no device): an
+    entry that sets a field takes the shape away from it, one that sets none
+    does not, and plan_get reports the persistent plan either way."""
+    Q.gemm_plan_clear()
+    try:
+        for kt in (True, False):
+            assert Q.gemm_is_small(256, 3072, 3072, k_tiled=kt)
+            assert not Q.gemm_is_small(4352, 12288, 3072, k_tiled=kt)
+            plan = Q.gemm_plan_get(256, 3072, 3072, k_tiled=kt)
+            Q.gemm_plan_set(256, 3072, 3072, k_tiled=kt)
+            assert Q.gemm_is_small(256, 3072, 3072, k_tiled=kt)
+            assert Q.gemm_plan_get(256, 3072, 3072, k_tiled=kt) == {**plan, "tuned": True}
+            for kw in (dict(group_m=4), dict(big_rows=0), dict(split=True), dict(tile=Q.PLAN_TILE_SQUARE)):
+                Q.gemm_plan_set(256, 3072, 3072, k_tiled=kt, **kw)
+                assert not Q.gemm_is_small(256, 3072, 3072, k_tiled=kt)
+        for bad in ((0, 3072, 3072), (256, 3072, 3072 + 64), (256, 3073, 3072), (1 << 40, 8, 256)):
+            assert not Q.gemm_is_small(*bad)
+    finally:
+        Q.gemm_plan_clear()
