@@ -1394,6 +1394,9 @@ void GemmTuneStore::apply() const {
 
 namespace {
 
+// An entry that sets no field: the library's own choice of kernel and plan.
+constexpr phi_gemm_plan kOwnChoice{-1, 0, 0, PHI_PLAN_TILE_AUTO, 0};
+
 // A shape's table entry taken out for a sweep and put back afterwards.
 struct PlanHold {
     i64 M, N, K;
@@ -1488,7 +1491,9 @@ GemmTuneResult autotune_int8_gemm(ComputeContext& ctx, i64 M, i64 N, i64 K, int 
         // Candidates: the square plan at the cost model's 256-row count and
         // its neighbours, all rows, group heights 2, 4, 8, and one or two
         // launches where both tile sizes run; with K % 512 == 0, also 272 x
-        // 192 tiles at each group height.
+        // 192 tiles at each group height.  Where the small-problem kernel takes
+        // the shape, the library's own choice first: every other candidate
+        // keeps that kernel out.
         phi_gemm_plan def{};
         ctx.check(phi_hip_gemm_plan_get(M, N, K, kt, &def, nullptr), "gemm_plan_get");
         std::vector<i64> rows_opts{def.big_rows};
@@ -1507,6 +1512,7 @@ GemmTuneResult autotune_int8_gemm(ComputeContext& ctx, i64 M, i64 N, i64 K, int 
             }
         } events{e0, e1};
         std::vector<phi_gemm_plan> cands;
+        if (phi_hip_gemm_is_small(M, N, K, kt)) cands.push_back(kOwnChoice);
         for (const i64 big : rows_opts)
             for (const int gm : {2, 4, 8})
                 for (const int split : {0, 1})

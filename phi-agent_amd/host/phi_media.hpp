@@ -464,7 +464,8 @@ LoraTail load_lora_tail(GpuCtx& g, GpuArena& arena, const std::string& base, con
 // (the square plan or 272 x 192 tiles, K % 512 == 0).  Every
 // plan gives the same bits, so a sweep is free to pick the fastest; it checks
 // that anyway.  The store persists as JSON and apply() hands its plans to the
-// library, whose every launch of such a shape then runs the stored plan.
+// library, whose every launch of such a shape then runs the stored plan.  A
+// shape that the small-problem kernel serves best is stored with no field set.
 struct GemmTuneEntry {
     i64 M = 0, N = 0, K = 0;
     bool k_tiled = false;

@@ -141,7 +141,8 @@ static int weights(int argc, char** argv) {
 }
 
 // autotune_int8_gemm, the winner stored and saved, the table cleared, the file
-// loaded into a new store and applied: the plan the library then runs.
+// loaded into a new store and applied: the plan the library then runs.  small:
+// whether the small-problem kernel then takes the shape.
 static int tune(char** argv) {
     const i64 M = atoll(argv[2]), N = atoll(argv[3]), K = atoll(argv[4]);
     const int iters = atoi(argv[5]);
@@ -161,10 +162,11 @@ static int tune(char** argv) {
     if (phi_hip_gemm_plan_get(M, N, K, kt ? 1 : 0, &p, &tuned) != PHI_OK) throw MediaError(phi_hip_last_error());
     printf("{\"ok\": true, \"default_exact\": %s, \"exact\": %d, \"tried\": %zu, \"best_us\": %.3f, "
            "\"best\": [%lld, %d, %d, %d], \"applied\": [%lld, %d, %d, %d], \"tuned\": %d, \"entries\": %zu, "
-           "\"us\": [",
+           "\"small\": %d, \"us\": [",
            r.default_exact ? "true" : "false", r.exact_matches, r.tried.size(), r.best.measured_us,
            (long long)r.best.big_rows, r.best.group_m, r.best.split ? 1 : 0, r.best.tile, (long long)p.big_rows,
-           (int)p.group_m, (int)p.split, (int)p.tile, tuned, back.size());
+           (int)p.group_m, (int)p.split, (int)p.tile, tuned, back.size(),
+           phi_hip_gemm_is_small(M, N, K, kt));
     for (size_t i = 0; i < r.tried.size(); i++) printf("%s%.3f", i ? ", " : "", r.tried[i].measured_us);
     printf("], \"tiles\": [");
     for (size_t i = 0; i < r.tried.size(); i++) printf("%s%d", i ? ", " : "", r.tried[i].tile);

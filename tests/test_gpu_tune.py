@@ -83,3 +83,20 @@ def test_autotune_sweep_round_trip(dev, tmp_path, kt, M, N, K):
         assert r["best"][3] in (Q.PLAN_TILE_SQUARE, Q.PLAN_TILE_272)
     else:
         assert r["best"][3] == Q.PLAN_TILE_SQUARE
+
+
+@pytest.mark.parametrize("kt", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(1, 3072, 3072), (256, 3072, 3072)])
+def test_autotune_small_problem(dev, tmp_path, kt, M, N, K):
+    """A problem that the small-problem kernel takes: the sweep times that too
+    (an entry that sets no field)."""
+    path = tmp_path / "gemm_plans.json"
+    r = json.loads(C.run("tune", M, N, K, 20, kt, str(path)).stdout)
+    assert r["ok"] and r["default_exact"] and r["exact"] == r["tried"]
+    assert r["tiles"].count(Q.PLAN_TILE_AUTO) == 1 and r["best_us"] == pytest.approx(min(r["us"]), rel=1e-6)
+    (e,) = json.loads(path.read_text())["plans"]
+    assert [e["big_rows"], e["group_m"], e["split"], e["tile"]] == r["best"]
+    own = r["best"][3] == Q.PLAN_TILE_AUTO
+    assert r["small"] == (1 if own else 0)
+    # It is far ahead here (2.7 and 1.5 times), beyond what runs differ by.
+    assert own and r["best"] == [-1, 0, 0, 0]
