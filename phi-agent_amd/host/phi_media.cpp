@@ -1397,7 +1397,9 @@ namespace {
 // An entry that sets no field: the library's own choice of kernel and plan.
 constexpr phi_gemm_plan kOwnChoice{-1, 0, 0, PHI_PLAN_TILE_AUTO, 0};
 
-// A shape's table entry taken out for a sweep and put back afterwards.
+// A shape's table entry taken out for a sweep and put back afterwards.  An
+// entry under which the small-problem kernel runs sets no field, and _get
+// reports every field set.
 struct PlanHold {
     i64 M, N, K;
     int kt;
@@ -1405,6 +1407,7 @@ struct PlanHold {
     int had = 0;
     PlanHold(i64 m, i64 n, i64 k, int t) : M(m), N(n), K(k), kt(t) {
         phi_hip_gemm_plan_get(M, N, K, kt, &saved, &had);
+        if (had && phi_hip_gemm_is_small(M, N, K, kt)) saved = kOwnChoice;
         phi_hip_gemm_plan_set(M, N, K, kt, nullptr);
     }
     ~PlanHold() { phi_hip_gemm_plan_set(M, N, K, kt, had ? &saved : nullptr); }

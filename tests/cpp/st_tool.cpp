@@ -140,16 +140,21 @@ static int weights(int argc, char** argv) {
     return 0;
 }
 
-// autotune_int8_gemm, the winner stored and saved, the table cleared, the file
-// loaded into a new store and applied: the plan the library then runs.  small:
-// whether the small-problem kernel then takes the shape.
+// autotune_int8_gemm beside a table entry that sets no field, the winner stored
+// and saved, the table cleared, the file loaded into a new store and applied:
+// the plan the library then runs.  small: whether the small-problem kernel
+// takes the shape before the sweep, after it, and with the winner applied.
 static int tune(char** argv) {
     const i64 M = atoll(argv[2]), N = atoll(argv[3]), K = atoll(argv[4]);
     const int iters = atoi(argv[5]);
     const bool kt = atoi(argv[6]) != 0;
     ComputeContext ctx(0);
+    const phi_gemm_plan own{-1, 0, 0, PHI_PLAN_TILE_AUTO, 0};
+    if (phi_hip_gemm_plan_set(M, N, K, kt, &own) != PHI_OK) throw MediaError(phi_hip_last_error());
+    const int small = phi_hip_gemm_is_small(M, N, K, kt);
     const GemmTuneResult r = autotune_int8_gemm(ctx, M, N, K, iters, kt);
     if (!r.ok) throw MediaError(r.error);
+    const int small_after = phi_hip_gemm_is_small(M, N, K, kt);
     GemmTuneStore store;
     store.put(r.best);
     if (!store.save(argv[7])) throw MediaError(std::string("cannot write ") + argv[7]);
@@ -162,11 +167,11 @@ static int tune(char** argv) {
     if (phi_hip_gemm_plan_get(M, N, K, kt ? 1 : 0, &p, &tuned) != PHI_OK) throw MediaError(phi_hip_last_error());
     printf("{\"ok\": true, \"default_exact\": %s, \"exact\": %d, \"tried\": %zu, \"best_us\": %.3f, "
            "\"best\": [%lld, %d, %d, %d], \"applied\": [%lld, %d, %d, %d], \"tuned\": %d, \"entries\": %zu, "
-           "\"small\": %d, \"us\": [",
+           "\"small\": [%d, %d, %d], \"us\": [",
            r.default_exact ? "true" : "false", r.exact_matches, r.tried.size(), r.best.measured_us,
            (long long)r.best.big_rows, r.best.group_m, r.best.split ? 1 : 0, r.best.tile, (long long)p.big_rows,
-           (int)p.group_m, (int)p.split, (int)p.tile, tuned, back.size(),
-           phi_hip_gemm_is_small(M, N, K, kt));
+           (int)p.group_m, (int)p.split, (int)p.tile, tuned, back.size(), small,
+           small_after, phi_hip_gemm_is_small(M, N, K, kt));
     for (size_t i = 0; i < r.tried.size(); i++) printf("%s%.3f", i ? ", " : "", r.tried[i].measured_us);
     printf("], \"tiles\": [");
     for (size_t i = 0; i < r.tried.size(); i++) printf("%s%d", i ? ", " : "", r.tried[i].tile);
