@@ -87,7 +87,7 @@ struct Shape {
 
 // Multiplier for dividing by a loop-invariant d >= 1: ceil(2^32 / d), which
 // is (2^32 - 1) / d + 1 for every d (0 for d = 1, handled in udiv_inv).
-__device__ __forceinline__ unsigned inv_mul(unsigned d) { return 0xffffffffu / d + 1u; }
+__host__ __device__ __forceinline__ unsigned inv_mul(unsigned d) { return 0xffffffffu / d + 1u; }
 
 // n / d for n < 2^32 with m = inv_mul(d): the high word of n * m is n / d or
 // one more (m exceeds 2^32 / d by less than 1, so n * m / 2^32 exceeds n / d

@@ -33,6 +33,7 @@
 // and sum rounds on its own, as the reference's x86-64 host code does).
 #include "device_common.hpp"
 #include "i8_gemm.hpp"
+#include "persist_common.hpp"
 #include "w4a8.hpp"
 
 namespace phi_dev {
@@ -69,41 +70,49 @@ __global__ __launch_bounds__(256) void dequant_rows_kernel(const void* src, int 
     }
 }
 
-// The same, four columns a thread and a row a block: 16-byte stores, the row's
-// scale read once, and no division (the one by `cols` for every element, in 64
-// bits, bound the general kernel: 12288 x 3072 int8 rows 81 us, this one 32
-// for 189 MB).  cols % 4 == 0, four elements of src and out aligned.
+// The same, four columns an item and two items a thread: 16-byte stores, and
+// 32-bit arithmetic to find an item's row (the 64-bit division by `cols` for
+// every element bound the general kernel: 12288 x 3072 int8 rows 81 us, this
+// one 32 for 189 MB).  Items run through all rows alike, so that narrow rows
+// fill their waves and a few wide ones spread over many blocks: with a row a
+// block, 2^20 rows of 4 columns took 224 us and 8 of 16384 5.2, here 5.3 and
+// 2.9.  cols % 4 == 0, four elements of src and out aligned; c4 = cols / 4,
+// mul = inv_mul(c4).
 template <int KIND>
-__global__ __launch_bounds__(256) void dequant_rows4_kernel(const void* __restrict__ src, int64_t rows, int64_t cols,
-                                                            int64_t lds, const float* __restrict__ row_scale,
-                                                            int scale_scalar, float* __restrict__ out, int64_t ldo) {
-    for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+__global__ __launch_bounds__(256) void dequant_rows4_kernel(const void* __restrict__ src, uint32_t items, uint32_t c4,
+                                                            uint32_t mul, int64_t lds,
+                                                            const float* __restrict__ row_scale, int scale_scalar,
+                                                            float* __restrict__ out, int64_t ldo) {
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const uint32_t i = (blockIdx.x * 2 + u) * 256 + threadIdx.x;
+        if (i >= items) return;
+        const uint32_t row = persist::udiv_inv(i, c4, mul);
+        const int64_t r = row, c = (int64_t)(i - row * c4) * 4;
         const float sc = row_scale ? row_scale[scale_scalar ? 0 : r] : 1.0f;
-        for (int64_t c = (int64_t)threadIdx.x * 4; c < cols; c += (int64_t)blockDim.x * 4) {
-            float v[4];
-            if (KIND == DQ_F32) {
-                const float4 t = *(const float4*)((const float*)src + r * lds + c);
-                v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
-            } else if (KIND == DQ_F16 || KIND == DQ_BF16) {
-                const uint2 t = *(const uint2*)((const uint16_t*)src + r * lds + c);
-                const uint32_t h[4] = {t.x & 0xffffu, t.x >> 16, t.y & 0xffffu, t.y >> 16};
+        float v[4];
+        if (KIND == DQ_F32) {
+            const float4 t = *(const float4*)((const float*)src + r * lds + c);
+            v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
+        } else if (KIND == DQ_F16 || KIND == DQ_BF16) {
+            const uint2 t = *(const uint2*)((const uint16_t*)src + r * lds + c);
+            const uint32_t h[4] = {t.x & 0xffffu, t.x >> 16, t.y & 0xffffu, t.y >> 16};
 #pragma unroll
-                for (int i = 0; i < 4; i++) v[i] = KIND == DQ_F16 ? f16_to_f32(h[i]) : bf16_to_f32(h[i]);
-            } else if (KIND == DQ_I4) {
-                const uint32_t t = *(const uint16_t*)((const uint8_t*)src + r * lds + (c >> 1));
+            for (int e = 0; e < 4; e++) v[e] = KIND == DQ_F16 ? f16_to_f32(h[e]) : bf16_to_f32(h[e]);
+        } else if (KIND == DQ_I4) {
+            const uint32_t t = *(const uint16_t*)((const uint8_t*)src + r * lds + (c >> 1));
 #pragma unroll
-                for (int i = 0; i < 4; i++) v[i] = (float)((int32_t)(t << (28 - 4 * i)) >> 28) * sc;
-            } else {
-                const uint32_t t = *(const uint32_t*)((const uint8_t*)src + r * lds + c);
+            for (int e = 0; e < 4; e++) v[e] = (float)((int32_t)(t << (28 - 4 * e)) >> 28) * sc;
+        } else {
+            const uint32_t t = *(const uint32_t*)((const uint8_t*)src + r * lds + c);
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t b = (t >> (8 * i)) & 0xffu;
-                    const float d = KIND == DQ_I8 ? (float)(int8_t)b : KIND == DQ_F8_E4M3 ? e4m3_to_f32(b) : e5m2_to_f32(b);
-                    v[i] = d * sc;
-                }
+            for (int e = 0; e < 4; e++) {
+                const uint32_t b = (t >> (8 * e)) & 0xffu;
+                const float d = KIND == DQ_I8 ? (float)(int8_t)b : KIND == DQ_F8_E4M3 ? e4m3_to_f32(b) : e5m2_to_f32(b);
+                v[e] = d * sc;
             }
-            *(float4*)(out + r * ldo + c) = make_float4(v[0], v[1], v[2], v[3]);
         }
+        *(float4*)(out + r * ldo + c) = make_float4(v[0], v[1], v[2], v[3]);
     }
 }
 
@@ -288,24 +297,33 @@ hipError_t launch_dequant_rows(hipStream_t stream, const void* src, int kind, in
                                const float* row_scale, int scale_scalar, float* out, int64_t ldo) {
     const int four = kind == DQ_F32 ? 16 : kind == DQ_F16 || kind == DQ_BF16 ? 8 : kind == DQ_I4 ? 2 : 4;  // bytes of four
     const int64_t pitch = kind == DQ_I4 ? lds : lds * (four / 4);
-    if (cols % 4 == 0 && (uintptr_t)src % four == 0 && pitch % four == 0 && (uintptr_t)out % 16 == 0 && ldo % 4 == 0) {
-        const dim3 grid((unsigned)(rows < (1 << 20) ? rows : 1 << 20)), block(cols >= 1024 ? 256 : cols >= 512 ? 128 : 64);
-#define PHI_DQ4(KIND)                                                                                              \
-    case KIND:                                                                                                     \
-        hipLaunchKernelGGL(dequant_rows4_kernel<KIND>, grid, block, 0, stream, src, rows, cols, lds, row_scale,     \
-                           scale_scalar, out, ldo);                                                                \
-        return hipGetLastError();
-        switch (kind) {
-            PHI_DQ4(DQ_I8)
-            PHI_DQ4(DQ_I4)
-            PHI_DQ4(DQ_F8_E4M3)
-            PHI_DQ4(DQ_F8_E5M2)
-            PHI_DQ4(DQ_F16)
-            PHI_DQ4(DQ_BF16)
-            PHI_DQ4(DQ_F32)
-            default: break;
-        }
+    const int64_t c4 = cols / 4, most = (int64_t)1 << 31;  // items a launch
+    if (cols % 4 == 0 && c4 <= most && (uintptr_t)src % four == 0 && pitch % four == 0 && (uintptr_t)out % 16 == 0 && ldo % 4 == 0) {
+        const uint32_t mul = persist::inv_mul((unsigned)c4);
+        for (int64_t r0 = 0; r0 < rows; r0 += most / c4) {
+            const uint32_t items = (uint32_t)((rows - r0 < most / c4 ? rows - r0 : most / c4) * c4);
+            const dim3 grid((items + 511) / 512), block(256);
+            const char* s = (const char*)src + r0 * pitch;
+            const float* sc = row_scale && !scale_scalar ? row_scale + r0 : row_scale;
+            float* o = out + r0 * ldo;
+#define PHI_DQ4(KIND)                                                                                                     \
+    case KIND:                                                                                                            \
+        hipLaunchKernelGGL(dequant_rows4_kernel<KIND>, grid, block, 0, stream, s, items, (uint32_t)c4, mul, lds, sc,       \
+                           scale_scalar, o, ldo);                                                                         \
+        break;
+            switch (kind) {
+                PHI_DQ4(DQ_I8)
+                PHI_DQ4(DQ_I4)
+                PHI_DQ4(DQ_F8_E4M3)
+                PHI_DQ4(DQ_F8_E5M2)
+                PHI_DQ4(DQ_F16)
+                PHI_DQ4(DQ_BF16)
+                PHI_DQ4(DQ_F32)
+                default: return hipErrorInvalidValue;
+            }
 #undef PHI_DQ4
+        }
+        return hipGetLastError();
     }
     hipLaunchKernelGGL(dequant_rows_kernel, dim3(grid_for(rows * cols)), dim3(256), 0, stream, src, kind, rows, cols,
                        lds, row_scale, scale_scalar, out, ldo);

@@ -26,7 +26,7 @@ def bits(t):
     return t.contiguous().view(torch.int32)
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 4), (3, 252), (5, 516), (2, 3076)])
+@pytest.mark.parametrize("rows,cols", [(1, 4), (3, 252), (5, 516), (2, 3076), (70001, 4), (300, 12), (129, 2048)])
 @pytest.mark.parametrize("kind", [Q.I8, Q.I4, Q.F8_E4M3, Q.F8_E5M2, Q.F16, Q.BF16, Q.F32])
 def test_dequant_rows(dev, kind, rows, cols):
     g = torch.Generator().manual_seed(cols)
