@@ -346,8 +346,13 @@ hipError_t launch_convrot_rows(hipStream_t stream, const float* x, int64_t ldx, 
 
 hipError_t launch_lora_fold(hipStream_t stream, float* w, int64_t ldw, int64_t rows, int64_t k, const float* A,
                             const float* B, int64_t rank, float scale) {
+    // The tiled form gives a wave 8 rows x 256 columns: below 768 K entries it
+    // leaves the chip emptier than one entry a thread does (64 x 3072 at rank 4:
+    // 4.0 against 3.7 us, 1024 x 256 at rank 64 16.9 against 16.3; from there on
+    // 256 x 3072 4.3 against 5.2, 3072 x 256 17.4 against 29.6), and below 64
+    // columns most of each wave (65536 x 32 at rank 64: 66 against 57).
     const int64_t cb = (k + 255) / 256, rb = (rows + 4 * LF_ROWS - 1) / (4 * LF_ROWS);
-    if (k % 4 == 0 && ldw % 4 == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)A % 16 == 0 && cb * rb <= INT32_MAX) {
+    if (k >= 64 && rows * k >= 3 << 18 && k % 4 == 0 && ldw % 4 == 0 && (uintptr_t)w % 16 == 0 && (uintptr_t)A % 16 == 0 && cb * rb <= INT32_MAX) {
         hipLaunchKernelGGL(lora_fold_tile_kernel, dim3((unsigned)(cb * rb)), dim3(256), 0, stream, w, ldw, rows, k, A, B,
                            rank, scale, (int)cb);
         return hipGetLastError();

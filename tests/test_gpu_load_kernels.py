@@ -57,7 +57,8 @@ def test_convrot_rows(dev, rows, K):
     assert torch.equal(torch.nan_to_num(inplace, nan=0.0), torch.nan_to_num(got, nan=0.0))
 
 
-@pytest.mark.parametrize("rows,k,rank", [(1, 4, 1), (63, 260, 4), (65, 516, 7), (130, 1024, 33)])
+@pytest.mark.parametrize("rows,k,rank", [(1, 4, 1), (63, 260, 4), (65, 516, 7), (130, 1024, 33), (12289, 64, 3), (3025, 260, 5),
+                                         (1031, 764, 33), (260, 3076, 4)])
 def test_lora_fold(dev, rows, k, rank):
     g = torch.Generator().manual_seed(rank)
     w, A, B = torch.randn(rows, k, generator=g), torch.randn(rank, k, generator=g), torch.randn(rows, rank, generator=g)
