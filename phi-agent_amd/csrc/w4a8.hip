@@ -15,11 +15,11 @@
 //   nibbles into the same int8 operand in registers (nibble4 only).
 //
 // Nibble codes in whole 16-byte chunks of one group each take
-// w4a8_table_kernel, one wave a row: a group has 16 possible values, so the
-// row needs 16 decodes a group and not one an element.  The general kernel
-// (packed6, other groups and alignments) runs one workgroup per row, each
-// thread decoding 16 consecutive columns at a time: pass 1 reduces the row
-// amax, pass 2 decodes again and quantises.
+// w4a8_table_kernel where that pays (w4a8_table_pays), one wave a row: a group
+// has 16 possible values, so the row needs 16 decodes a group and not one an
+// element.  The general kernel (packed6, other groups and alignments) runs one
+// workgroup per row, each thread decoding 16 consecutive columns at a time:
+// pass 1 reduces the row amax, pass 2 decodes again and quantises.
 #include "device_common.hpp"
 #include "persist_common.hpp"
 #include "w4a8.hpp"
@@ -217,6 +217,25 @@ __global__ __launch_bounds__(256) void w4a8_table_kernel(W4a8Params p, int8_t* _
     }
 }
 
+// Where the table kernel beats the general one (189 sizes a function).  Its
+// LDS holds 84 bytes a group and wave: above 240 groups one block fits a CU.
+// With groups of 32 the general kernel, which spreads a row over four waves,
+// is then as fast where there are rows enough to fill the chip otherwise
+// (expand, 3072 rows x 8192: 138 us against 121).  Prepare decodes each table
+// entry, half the work of an element's in expand, so the line lies lower: with
+// few rows a wave's own chain bounds it, 16 entries a group, where the general
+// kernel takes a step of 4096 columns (256 x 3072 in groups of 32, 96 of them:
+// 14 us against 10); with many, two blocks a CU (3072 x 6144, 192 groups: 74
+// against 58; 160 groups 30 against 54).  Groups of 128 and up have few
+// entries a column: never.
+static bool w4a8_table_pays(const W4a8Params& p, bool lut) {
+    const int64_t G = p.k / p.group;
+    if (!lut) return G <= 240 || p.group >= 64 || p.rows <= 2048;
+    if (p.group >= 128) return true;
+    if (p.rows < 1024) return G <= 60 * ((p.k + 4095) / 4096);
+    return G <= 160 || (p.group >= 64 && p.rows <= 2048);
+}
+
 // The table kernel's limits: 16-byte code chunks that lie in one group, and
 // four rows' tables in LDS.
 static bool w4a8_table_ok(const W4a8Params& p) {
@@ -237,7 +256,7 @@ static hipError_t launch_table(hipStream_t stream, const W4a8Params& p, int8_t* 
 }
 
 hipError_t launch_w4a8_rows(hipStream_t stream, const W4a8Params& p, int8_t* out, float* s, bool lut) {
-    if (w4a8_table_ok(p)) return lut ? launch_table<true>(stream, p, out, s) : launch_table<false>(stream, p, out, s);
+    if (w4a8_table_ok(p) && w4a8_table_pays(p, lut)) return lut ? launch_table<true>(stream, p, out, s) : launch_table<false>(stream, p, out, s);
     if (lut)
         hipLaunchKernelGGL(w4a8_rows_kernel<true>, dim3((unsigned)p.rows), dim3(256), 0, stream, p, out, s);
     else

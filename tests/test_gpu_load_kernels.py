@@ -79,7 +79,8 @@ def test_lora_fold(dev, rows, k, rank):
 
 
 @pytest.mark.parametrize("with_cb", [False, True])
-@pytest.mark.parametrize("rows,k,group", [(1, 32, 32), (5, 1056, 32), (7, 3072, 128), (2, 15360, 32), (3, 4096, 4096)])
+@pytest.mark.parametrize("rows,k,group", [(1, 32, 32), (5, 1056, 32), (7, 3072, 128), (2, 15360, 32), (3, 4096, 4096), (3, 1920, 32), (3, 1952, 32),
+                                          (1025, 5120, 32), (2049, 7680, 32), (2049, 7712, 32)])
 def test_w4a8_expand_and_prepare(dev, rows, k, group, with_cb):
     codes, s_rel, sch, corr = (t.to(dev) for t in synth.w4a8_weight(rows, k, group, seed=rows))
     codes[0] &= 0x33  # a row that uses only some of the codes
