@@ -291,6 +291,102 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
     }
 }
 
+// The same chains on v_fmac_f32, one row a lane, for few columns or ranks: the
+// kernel above always runs its 16-rank tiles over eight chunks' loads, with a
+// block or two a CU; here a block (64 rows, a wave two ranks) needs 36 KB of
+// LDS and few registers, and four fit a CU.  Each 64-k chunk of the rows' x and
+// of the waves' A slices goes global -> registers -> LDS, double-buffered with
+// one barrier a chunk, the next chunk's global loads in flight under the
+// current chunk's fmas.  A lane reads its own row of x (68-float pitch: 16-byte
+// aligned rows, conflict-free 16-byte reads and writes) and its wave's A
+// values, which all the wave's lanes read at one address (a broadcast).
+// 100000 x 64 x 4 fp32: 6.3 us, above 16.9; 4352 x 64 x 64 5.7 against 7.1.
+constexpr int LR_TR = 2;
+
+// 64 rows x 64 k of x into registers: lane t holds row t / 4, k 16 (t % 4)..+15.
+template <bool XB>
+__device__ __forceinline__ void fetch_x_tile(const void* __restrict__ x, int64_t ldx, int m0, int M, int k0,
+                                             float (&v)[16]) {
+    const int row = threadIdx.x >> 2, kk = (threadIdx.x & 3) * 16;
+    const int64_t off = (int64_t)min(m0 + row, M - 1) * ldx + k0 + kk;
+    if (XB) {
+        const uint4 a = *(const uint4*)((const uint16_t*)x + off), b = *(const uint4*)((const uint16_t*)x + off + 8);
+        const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            v[2 * i] = bf16_to_f32(w[i] & 0xffffu);
+            v[2 * i + 1] = bf16_to_f32(w[i] >> 16);
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 t = *(const float4*)((const float*)x + off + 4 * q);
+            v[4 * q] = t.x, v[4 * q + 1] = t.y, v[4 * q + 2] = t.z, v[4 * q + 3] = t.w;
+        }
+    }
+}
+
+// x rows 16-byte aligned, K % 64 == 0.
+template <bool XB>
+__global__ __launch_bounds__(256) void lora_down_rows_kernel(const void* __restrict__ x, int64_t ldx,
+                                                             const float* __restrict__ A, float* __restrict__ h,
+                                                             int M, int K, int R) {
+    __shared__ __align__(16) float sx[2][64 * LD_P];
+    __shared__ __align__(16) float sa[2][4][LR_TR * LD_KC];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m0 = blockIdx.x * 64;
+    const int rb = (blockIdx.y * 4 + wave) * LR_TR;
+    const bool live = rb < R;  // wave-uniform; a dead wave still stages x for the others
+    // The wave's A slice of a chunk (LR_TR ranks x 64 k, rank-major): lane l
+    // holds LR_TR consecutive k of rank l / LPR.  Ranks past R read rank R - 1.
+    constexpr int LPR = LD_KC / LR_TR;
+    const int at = lane / LPR, ak = (lane % LPR) * LR_TR;
+    const float* arow = A + (int64_t)min(rb + at, R - 1) * K + ak;
+    float acc[LR_TR] = {0.0f, 0.0f};
+    float xt[16];
+    fetch_x_tile<XB>(x, ldx, m0, M, 0, xt);
+    float2 ta = *(const float2*)arow;
+    const int srow = threadIdx.x >> 2, skk = (threadIdx.x & 3) * 16;
+    for (int k0 = 0, buf = 0; k0 < K; k0 += LD_KC, buf ^= 1) {
+        float* st = sx[buf] + srow * LD_P + skk;
+#pragma unroll
+        for (int q = 0; q < 4; q++) *(float4*)(st + 4 * q) = make_float4(xt[4 * q], xt[4 * q + 1], xt[4 * q + 2], xt[4 * q + 3]);
+        *(float2*)&sa[buf][wave][at * LD_KC + ak] = ta;
+        __syncthreads();
+        if (k0 + LD_KC < K) {
+            fetch_x_tile<XB>(x, ldx, m0, M, k0 + LD_KC, xt);
+            ta = *(const float2*)(arow + k0 + LD_KC);
+        }
+        if (live) {
+            const float* xr = sx[buf] + lane * LD_P;
+            const float* as = sa[buf][wave];
+#pragma unroll
+            for (int kk = 0; kk < LD_KC; kk += 8) {
+                const float4 x0 = *(const float4*)(xr + kk), x1 = *(const float4*)(xr + kk + 4);
+                const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+                float av[LR_TR][8];
+#pragma unroll
+                for (int t = 0; t < LR_TR; t++) {
+                    const float4 a0 = *(const float4*)(as + t * LD_KC + kk), a1 = *(const float4*)(as + t * LD_KC + kk + 4);
+                    av[t][0] = a0.x, av[t][1] = a0.y, av[t][2] = a0.z, av[t][3] = a0.w;
+                    av[t][4] = a1.x, av[t][5] = a1.y, av[t][6] = a1.z, av[t][7] = a1.w;
+                }
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+#pragma unroll
+                    for (int t = 0; t < LR_TR; t++) acc[t] = fmaf(xv[i], av[t][i], acc[t]);
+            }
+        }
+        // The buffer written next iteration was last read two iterations ago,
+        // before this iteration's barrier: one barrier per chunk suffices.
+    }
+    const int m = m0 + lane;
+    if (!live || m >= M) return;
+#pragma unroll
+    for (int t = 0; t < LR_TR; t++)
+        if (rb + t < R) h[(int64_t)m * R + rb + t] = acc[t];  // K % 32 == 0: no padding
+}
+
 template <bool XB, bool VEC, int WR, int RT>
 static hipError_t launch_down(hipStream_t stream, const void* x, int64_t ldx, const float* A, float* h, int M, int K,
                               int R) {
@@ -304,13 +400,14 @@ static hipError_t launch_down(hipStream_t stream, const void* x, int64_t ldx, co
 // wave of a block idles and x is read as few times as possible.  One chain a
 // wave while every chain finds a SIMD of its own (4 a CU), two beyond: the
 // pair takes as long as two chains on one SIMD would, and A is read half as
-// often.
+// often.  Up to 16 ranks x is what the time goes to, and one chain a wave (two
+// blocks a CU and not one) is the faster at any size: 65536 x 3072 x 16 163
+// against 176 us, 100000 x 512 x 16 43 against 63.
 template <bool XB, bool VEC>
 static hipError_t launch_down_r(hipStream_t stream, const void* x, int64_t ldx, const float* A, float* h, int M, int K,
                                 int R) {
     const bool one = ((int64_t)M + 15) / 16 * ((R + 15) / 16) <= 1024;
-    if (R <= 16) return one ? launch_down<XB, VEC, 1, 1>(stream, x, ldx, A, h, M, K, R)
-                            : launch_down<XB, VEC, 1, 2>(stream, x, ldx, A, h, M, K, R);
+    if (R <= 16) return launch_down<XB, VEC, 1, 1>(stream, x, ldx, A, h, M, K, R);
     if (R <= 32) return one ? launch_down<XB, VEC, 2, 1>(stream, x, ldx, A, h, M, K, R)
                             : launch_down<XB, VEC, 2, 2>(stream, x, ldx, A, h, M, K, R);
     return one ? launch_down<XB, VEC, 4, 1>(stream, x, ldx, A, h, M, K, R)
@@ -320,6 +417,17 @@ static hipError_t launch_down_r(hipStream_t stream, const void* x, int64_t ldx, 
 hipError_t launch_lora_down(hipStream_t stream, const void* x, bool x_bf16, int64_t ldx, const float* A, float* h,
                             int M, int K, int R) {
     const int esz = x_bf16 ? 2 : 4;
+    // One row a lane: a chunk or two of columns, and few ranks of many rows
+    // (measured against the tiles over 1130 sizes: 32760 x 1024 x 4 fp32 21.7
+    // against 26.4 us, 4352 x 64 x 16 4.0 against 5.1; 4352 x 256 x 64 10.7
+    // against 8.5, 32760 x 2048 x 16 80 against 47).
+    if ((K <= 64 || (R <= 16 && K <= 192) || (R <= 8 && M > 16384 && K <= 1024)) && K % LD_KC == 0 &&
+        (uintptr_t)x % 16 == 0 && (ldx * esz) % 16 == 0 && (uintptr_t)A % 16 == 0) {
+        const dim3 grid((unsigned)(((int64_t)M + 63) / 64), (unsigned)((R + 4 * LR_TR - 1) / (4 * LR_TR)));
+        if (x_bf16) hipLaunchKernelGGL(lora_down_rows_kernel<true>, grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
+        else hipLaunchKernelGGL(lora_down_rows_kernel<false>, grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
+        return hipGetLastError();
+    }
     const bool vec = K % 4 == 0 && ldx % 4 == 0 && (uintptr_t)x % (4 * esz) == 0 && (uintptr_t)A % 16 == 0;
     if (x_bf16) return vec ? launch_down_r<true, true>(stream, x, ldx, A, h, M, K, R)
                            : launch_down_r<true, false>(stream, x, ldx, A, h, M, K, R);

@@ -165,3 +165,19 @@ def test_lora_tiles_bit_exact(dev, orc, cdt, M, K, N, R):
         assert np.array_equal(bits(y), want.view(np.int32))
     else:
         assert torch.equal(y.cpu().view(torch.int16), torch.from_numpy(want).to(torch.bfloat16).view(torch.int16))
+
+
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,K,R", [(1, 64, 1), (65, 64, 17), (129, 64, 130), (64, 128, 16), (70, 192, 9), (70, 192, 17),
+                                   (16384, 256, 8), (16385, 256, 8), (16385, 1024, 3), (16385, 256, 9)])
+def test_lora_down_one_row_a_lane(dev, orc, xdt, M, K, R):
+    """Both sides of the lines between the chains of one row a lane and the
+    matrix-core tiles: few columns, or few ranks of many rows."""
+    x, A, _, _ = factors(M, K, R, 1, M + 3 * K + R)
+    x[0] *= 1e-38
+    x[-1] = -0.0
+    A[:, ::3] = 0.0
+    x = x.to(xdt)
+    h = Q.lora_down(x.to(dev), A.to(dev))
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(h), orc.lora_down(x.float().numpy(), A.numpy()).view(np.int32))
