@@ -46,7 +46,8 @@ def test_lora_down_bit_exact(dev, orc, monkeypatch, tr, xdt, M, K, R):
 
 
 @pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("M,N,R", [(1, 1, 1), (37, 1000, 17), (300, 513, 64), (129, 256, 256), (200, 130, 33)])
+@pytest.mark.parametrize("M,N,R", [(1, 1, 1), (37, 1000, 17), (300, 513, 64), (129, 256, 256), (200, 130, 33), (131, 644, 16),
+                                   (70, 1300, 5), (70, 1300, 17)])
 def test_lora_rank_add_bit_exact(dev, orc, cdt, M, N, R):
     g = torch.Generator().manual_seed(M * N + R)
     h = torch.randn(M, R, generator=g)
