@@ -29,17 +29,20 @@ def bits(t):
     return t.cpu().contiguous().view(torch.int32).numpy()
 
 
-@pytest.mark.parametrize("tr", ["1", "2", "4"])
+# Ranks around 16, 32 and 64 (one, two or four waves over them), one chain a
+# wave and two (above 1024 16 x 16 tiles: 8192 rows of 32 ranks, 4096 of 64),
+# rows that allow four-column loads and rows that do not (K or the pitch odd).
+@pytest.mark.parametrize("pad", [0, 1])
 @pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M,K,R", [(1, 256, 1), (37, 72, 17), (300, 3072, 64), (129, 1000, 256), (65, 33, 33),
-                                   (70, 640, 37)])
-def test_lora_down_bit_exact(dev, orc, monkeypatch, tr, xdt, M, K, R):
-    """tr: ranks per wave of the main form (the PHI_LORA_TR A/B switch); the
-    shapes with K % 64 == 0 take the main form, the others the general one."""
-    monkeypatch.setenv("PHI_LORA_TR", tr)
+                                   (70, 640, 37), (130, 260, 16), (130, 260, 32), (130, 260, 65), (8192, 200, 32),
+                                   (8193, 200, 32), (4096, 200, 64), (4097, 200, 64), (4097, 200, 40)])
+def test_lora_down_bit_exact(dev, orc, xdt, pad, M, K, R):
     x, A, _, _ = factors(M, K, R, 1, M + K + R)
     x = x.to(xdt)
-    h = Q.lora_down(x.to(dev), A.to(dev))
+    wide = torch.zeros((M, K + pad), dtype=xdt, device=dev)
+    wide[:, :K] = x.to(dev)
+    h = Q.lora_down(wide[:, :K], A.to(dev))
     torch.cuda.synchronize()
     want = orc.lora_down(x.float().numpy(), A.numpy())
     assert np.array_equal(bits(h), want.view(np.int32))
@@ -128,8 +131,8 @@ def test_lora_tail_full_size_rows_sampled(dev, orc):
 
 
 def test_lora_down_both_forms_agree(dev, orc):
-    """16-byte aligned rows take the row-streaming kernel; a row base 4 bytes in
-    takes the LDS-tiled one.  Both run the same chains."""
+    """Rows whose base and pitch allow four-column loads, and the same rows 4
+    bytes further on at an odd pitch (one element a load)."""
     M, K, R = 130, 512, 40
     x, A, _, _ = factors(M, K + 1, R, 1, 77)
     A = A[:, :K].contiguous()
@@ -182,3 +185,38 @@ def test_lora_down_one_row_a_lane(dev, orc, xdt, M, K, R):
     h = Q.lora_down(x.to(dev), A.to(dev))
     torch.cuda.synchronize()
     assert np.array_equal(bits(h), orc.lora_down(x.float().numpy(), A.numpy()).view(np.int32))
+
+
+def same_values(got, want):
+    """The same bits, NaN payloads and signs aside."""
+    g, w = got.float().cpu().numpy(), np.asarray(want, dtype=np.float32)
+    nan = np.isnan(w)
+    return np.array_equal(np.isnan(g), nan) and np.array_equal(g.view(np.int32)[~nan], w.view(np.int32)[~nan])
+
+
+# The matrix-core tiles (K > 64, R > 16: one and two chains a wave, with and
+# without four-column loads) and the chains of one row a lane (K = 64).
+@pytest.mark.parametrize("M,K,R", [(40, 328, 20), (40, 333, 20), (8200, 324, 20), (40, 64, 20)])
+def test_lora_tail_non_finite(dev, orc, M, K, R):
+    """Infinities, NaN, and chains that overflow on the way, in both passes."""
+    N = 132
+    x, A, B, out = factors(M, K, R, N, K)
+    inf, big = float("inf"), 3e38
+    x[1, 5], x[2, K - 1], x[M - 2, 3] = inf, float("nan"), -inf
+    x[3, 0], x[3, 9] = inf, -inf          # NaN unless A's signs differ
+    x[4, :4] = big
+    A[3, :4] = 2.0                        # overflows to inf, then meets -inf
+    A[4, :4] = torch.tensor([0.5, 0.5, 0.5, -0.5])
+    A[6], A[7, 2] = 0.0, inf              # 0 * inf; finite * inf
+    x[5], A[8] = 1e30, 1e10               # every product overflows
+    B[2, 1], B[3, 0], B[5], B[9, R - 1] = inf, float("nan"), 0.0, -inf
+    out[6], out[7, ::2], out[8, 3] = inf, -inf, float("nan")
+    B[11], out[9] = 1e30, -big
+    y = out.to(dev)
+    h = torch.empty((M, R), dtype=torch.float32, device=dev)
+    Q.lora_tail(x.to(dev), A.to(dev), B.to(dev), y, h=h)
+    torch.cuda.synchronize()
+    hw = orc.lora_down(x.numpy(), A.numpy())
+    assert np.isinf(hw).any() and np.isnan(hw).any() and same_values(h, hw)
+    want = orc.lora_rank_add(hw, B.numpy(), out.numpy())
+    assert np.isinf(want).any() and same_values(y, want)
