@@ -261,18 +261,30 @@ bool use_t272(const phi_dev::GemmParams& p, int G, int tile) {
     return t < square_plan_cost(p.M, p.N, G) - 1e-9;
 }
 
-// Below what a problem takes on the persistent kernels, in us: its rounds of
-// tiles at the fastest K-step measured (a round of 128 x 128 tiles with most
-// CUs idle; W4 codes expanded in registers: a full round of 256 x 256), one
-// pass over the operands, and the launch.
+// Rounds of tiles p takes on the persistent int8 kernels.
+double plan_rounds(const phi_dev::GemmParams& p, int G) {
+    const double rounds = square_plan_cost(p.M, p.N, G);
+    if (!phi_dev::t272_ok(p)) return rounds;
+    return std::min(rounds, (p.kt ? (p.b_rm ? kT272RoundMixed : kT272Round) : kT272RoundRowMajor) *
+                                (double)((phi_dev::t272_tile_count(p.M, p.N) + G - 1) / G));
+}
+
+// GB of operands through LDS, counted as 128 x 128 tiles.
+double lds_gb(const phi_dev::GemmParams& p) { return ceil(p.M / 128.0) * ceil(p.N / 128.0) * 256e-9 * p.K; }
+
+// What a problem takes on the persistent kernels, in us: the launch, its rounds
+// of tiles (a round of 128 x 128 tiles with most CUs idle), its operands from
+// memory and through LDS, and its outputs.  Fitted over 1700 random shapes of up
+// to 8 M outputs, the weight in cache and not, to their geometric mean: rms
+// error 8 %.  w4: codes expanded in registers, signed nibbles (6 %) or through
+// tables (8 %, the weight in cache).
 double persist_us(const phi_dev::GemmParams& p, bool w4, int G) {
-    double rounds = square_plan_cost(p.M, p.N, G);
-    if (!w4 && phi_dev::t272_ok(p))
-        rounds = std::min(rounds, (p.kt ? (p.b_rm ? kT272RoundMixed : kT272Round) : kT272RoundRowMajor) *
-                                      (double)((phi_dev::t272_tile_count(p.M, p.N) + G - 1) / G));
-    const double steps = rounds * (p.K / 64), mb = ((double)p.N + p.M) * p.K / 1e6;
-    if (w4) return 4.0 + 1.05 * steps;
-    return p.kt ? 3.6 + 0.42 * steps + 0.15 * mb : 3.6 + 0.45 * steps + 0.20 * mb;
+    const double steps = (w4 ? square_plan_cost(p.M, p.N, G) : plan_rounds(p, G)) * (p.K / 64), out = 1e-6 * p.M * p.N;
+    if (w4 && p.w4_signed) return 4.8 + 1.09 * steps + 0.09e-6 * p.N * p.K + 0.77 * out;
+    if (w4) return 4.15 + 1.37 * steps + 20.0 * lds_gb(p) + 0.56 * out;
+    const bool wide = p.c_kind != phi_dev::C_BF16;
+    return 4.0 + (p.gate ? 0.9 : wide ? 0.7 : 0.0) + (p.kt ? 0.448 : 0.488) * steps + 0.033e-6 * ((double)p.N + p.M) * p.K +
+           (p.kt ? 22.9 : 30.4) * lds_gb(p) + (p.gate ? 0.79 : wide ? 0.45 : 0.34) * out;
 }
 
 // The same of the register-staged tile kernels (gemm_kernel_for, gemm_cfg_for).
@@ -284,13 +296,14 @@ double tile_us(const phi_dev::GemmParams& p, int G) {
 }
 
 // The same of W4A8 with per-group tables: expanded once into a workspace, in
-// LDS on the 272 x 192 pipeline, or in registers.
+// LDS on the 272 x 192 pipeline, or in registers (970 shapes, rms error 6 to 8 %).
 double w4a8_us(const phi_dev::GemmParams& p, int G, bool workspace) {
     phi_dev::GemmParams q = p;
     q.kt = 1;
-    if (workspace) return persist_us(q, false, G) + 0.30 * (double)p.N * p.K / 1e6;
+    const double out = 1e-6 * p.M * p.N;
+    if (workspace) return 4.1 + 0.533 * plan_rounds(q, G) * (p.K / 64) + 0.4e-6 * p.N * p.K + 7.0 * lds_gb(p) + 0.99 * out;
     if (p.K > 16384 || !phi_dev::t272w4_ok(q)) return persist_us(p, true, G);
-    return 4.0 + 0.7 * ceil((double)phi_dev::t272_tile_count(p.M, p.N) / G) * (p.K / 64);
+    return 9.8 + 0.645 * ceil((double)phi_dev::t272_tile_count(p.M, p.N) / G) * (p.K / 64) + 20.0 * lds_gb(p) + 0.67 * out;
 }
 
 // The small-problem kernel's tile for p where the model says it beats
@@ -301,12 +314,12 @@ int skinny_choice(const phi_dev::GemmParams& p, bool w4, int G, double other_us)
     if (!phi_dev::skinny_ok(p, w4)) return -1;
     if (getenv("PHI_GEMM_KERNEL") || getenv("PHI_GEMM_PIPE") || getenv("PHI_GEMM_MIXED") || getenv("PHI_GEMM_T272")) return -1;
     if (getenv("PHI_GEMM_SKINNY")) return phi_dev::env_switch("PHI_GEMM_SKINNY", -1, 0, phi_dev::skinny_configs() - 1);
-    // The margin is the model's error: over 150 random shapes nothing it takes
-    // got slower, and half got more than 2.2 times faster (one row on 3072 ->
-    // 3072: 12.5 -> 4.6 us, 4096 rows onto 64 columns: 11.5 -> 4.8).
+    // The margin is the models' error.  Over 1155 other random shapes (every
+    // route that comes here, up to 30 M outputs) 877 got faster by more than 4 %,
+    // to 0.37 of the time in the geometric mean, and two slower, by 5 and 7 %.
     double us;
     const int cfg = phi_dev::skinny_best(p, w4, G, &us);
-    return 1.15 * us + 0.5 < other_us ? cfg : -1;
+    return 1.1 * us + 0.3 < other_us ? cfg : -1;
 }
 
 // Whether a problem the persistent kernel refuses only for its output (pieces
@@ -323,12 +336,13 @@ bool loose_ok(const phi_dev::GemmParams& p, bool pok, bool staged_ok) {
            phi_dev::env_switch("PHI_GEMM_LOOSE", 1, 0, 1);
 }
 
-// The same as persist_us for it: its stores cost a round about 10 us.  Against
+// The same as persist_us for it.  Against
 // the register-staged tiles: 4096 x 4101 x 3072 in bf16 139 -> 94 us, 8000 x
 // 11645 x 1024 in fp32 384 -> 261, 2000 x 1001 x 2048 26 -> 17 (whole pieces
 // take 58, 200 and 9).
 double loose_us(const phi_dev::GemmParams& p, int G) {
-    return persist_us(p, false, G) + 3.0 + 10.0 * square_plan_cost(p.M, p.N, G);
+    const double rounds = square_plan_cost(p.M, p.N, G);
+    return 3.6 + rounds * (12.9 + 0.508 * (p.K / 64)) + 0.01e-6 * ((double)p.N + p.M) * p.K + 33.7 * lds_gb(p) + 1.0e-6 * p.M * p.N;
 }
 
 // Whether a tuning-table entry says how the persistent kernel runs (and not

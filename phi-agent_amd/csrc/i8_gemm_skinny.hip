@@ -221,32 +221,61 @@ __device__ __forceinline__ void skinny_tile(const GemmParams& p, int8_t* smem) {
 
 // The tiles the kernel is built for: wave tile, waves a block, stages a wave.
 // More waves beat more stages a wave (4 x 4 tiles over K = 12288 at 256 rows:
-// 26.3 us with 8 waves of one stage, 27.0 with 4 of two).
+// 26.3 us with 8 waves of one stage, 27.0 with 4 of two).  Then, as fitted (see
+// skinny_us), in us by what B is (SkinnyB): the tile's part of the fixed time,
+// and what a round of blocks takes for a 128-column pair and apart from its
+// pairs.
 struct SkinnyCfg {
     int mt, nt, nw, s;
+    double fixed[3], pair[3], block[3];
 };
-constexpr SkinnyCfg kSkinny[] = {{1, 1, 8, 2}, {1, 2, 8, 1}, {1, 4, 8, 1}, {2, 1, 8, 1}, {2, 2, 8, 1}, {2, 4, 8, 1},
-                                 {4, 1, 8, 1}, {4, 2, 8, 1}, {4, 4, 8, 1}, {5, 2, 8, 1}, {5, 4, 8, 1}, {6, 4, 4, 2},
-                                 {3, 8, 4, 1}, {5, 8, 4, 1}};
+constexpr SkinnyCfg kSkinny[] = {
+    {1, 1, 8, 2, {0.59, 0.13, 0.73}, {0.0345, 0.0476, 0.0254}, {0.45, 0.45, 0.29}},
+    {1, 2, 8, 1, {0.99, 0.52, 1.00}, {0.0533, 0.0895, 0.0411}, {0.10, 0.07, 0.13}},
+    {1, 4, 8, 1, {1.16, 0.61, 1.20}, {0.0917, 0.1810, 0.0681}, {0.16, 0.09, 0.11}},
+    {2, 1, 8, 1, {0.97, 0.57, 0.99}, {0.0492, 0.0521, 0.0386}, {0.15, 0.21, 0.18}},
+    {2, 2, 8, 1, {0.98, 0.61, 1.08}, {0.0699, 0.0914, 0.0506}, {0.25, 0.26, 0.21}},
+    {2, 4, 8, 1, {0.13, 1.11, 1.25}, {0.1170, 0.1797, 0.0874}, {1.47, 0.00, 0.28}},
+    {4, 1, 8, 1, {1.05, 0.75, 0.91}, {0.0821, 0.0851, 0.0727}, {0.32, 0.30, 0.50}},
+    {4, 2, 8, 1, {0.15, 0.09, 1.21}, {0.1073, 0.1370, 0.0870}, {1.48, 1.17, 0.44}},
+    {4, 4, 8, 1, {0.00, 0.42, 0.15}, {0.1666, 0.2422, 0.1438}, {2.11, 1.31, 2.00}},
+    {5, 2, 8, 1, {0.14, 0.16, 0.00}, {0.1277, 0.1617, 0.1151}, {1.77, 1.43, 1.97}},
+    {5, 4, 8, 1, {0.19, 0.71, 0.28}, {0.1880, 0.2646, 0.1744}, {2.23, 1.37, 2.28}},
+    {6, 4, 4, 2, {0.24, 0.44, 0.53}, {0.2088, 0.3776, 0.2304}, {3.23, 2.23, 3.21}},
+    {3, 8, 4, 1, {0.42, 0.31, 0.52}, {0.2332, 0.4556, 0.2131}, {3.49, 2.48, 3.22}},
+    {5, 8, 4, 1, {0.52, 1.86, 0.80}, {0.2641, 0.5525, 0.3079}, {5.67, 2.98, 5.17}},
+};
 constexpr int kSkinnyCfgs = (int)(sizeof kSkinny / sizeof kSkinny[0]);
 
 int skinny_configs() { return kSkinnyCfgs; }
 
-// Time of p on tile cfg in us: a fixed part, then the larger of the weight's
-// one pass from memory and the busiest CU's blocks, each its operands' bytes
-// at a CU's rate into LDS plus a part that grows with the tile (the fill, the
-// sum over waves, the stores).  Fitted over 90 shapes x 12 tiles (one to 2048
-// rows, 64 to 12288 columns, K 1024 to 12288, both layouts; rms error 15 %):
-// the tile it picks is within 1 % of the best on average, 12 % at worst.
+// Time of p on tile cfg in us: a fixed part, the rounds of blocks and the
+// operands' pass from memory (the weight once; A once a column panel, rows
+// first, unless the L2s hold it) as the two sides of a right triangle, for they
+// overlap and disturb each other, the weight's share of a first pass, and the
+// stores.  Fitted over 2400 random shapes x 14 tiles (1 to 16384 rows, 8 to
+// 40000 columns, K 512 to 16384, both layouts, every output), the weight in
+// cache and not, to their geometric mean, rms error 7 % (signed nibbles 6 %);
+// codes through tables over 970 shapes with the weight in cache, 10 %.  On 630
+// other int8 and nibble shapes the error is 7 %, and the tile it picks within
+// 0.8 % of the best on average, within 5 % on 95 of 100.
 static double skinny_us(const GemmParams& p, bool w4, int num_cus, int cfg) {
     const SkinnyCfg c = kSkinny[cfg];
-    const double blocks = (double)((p.M + 16 * c.mt - 1) / (16 * c.mt)) * (double)((p.N + 16 * c.nt - 1) / (16 * c.nt));
-    const double rounds = ceil(blocks / num_cus), pairs = p.K / 128.0, weight = (double)p.N * p.K * (w4 ? 0.5 : 1.0);
-    const double kb = pairs * (2.0 * c.mt + (!w4 ? 2.0 : p.w4_signed ? 1.0 : 1.5) * c.nt);
-    if (w4 && !p.w4_signed)
-        return 2.6 + fmax(rounds * (kb * 0.0097 + pairs * c.nt * 0.027 + 0.180 * c.mt * c.nt), weight / 2.1e6);
-    if (w4) return 2.8 + fmax(rounds * (kb * 0.0080 + 0.234 * c.mt * c.nt + 0.11), weight / 5.6e6);
-    return 2.0 + fmax(rounds * (kb * 0.01326 + 0.139 * c.mt * c.nt + 0.16), weight / 4.1e6);
+    const int b = !w4 ? SB_I8 : p.w4_signed ? SB_S4 : SB_LUT;
+    const double tiles_m = (p.M + 16 * c.mt - 1) / (16 * c.mt), tiles_n = (p.N + 16 * c.nt - 1) / (16 * c.nt);
+    const double rounds = ceil(tiles_m * tiles_n / num_cus), pairs = p.K / 128.0, out = 1e-6 * p.M * p.N;
+    const double weight = 1e-6 * p.N * p.K * (w4 ? 0.5 : 1.0), a = 1e-6 * p.M * p.K;
+    // By what B is: fixed, a MB from memory, a MB of the weight, a million
+    // outputs, and a 16 x 16 tile of a block's.
+    constexpr double kUs[3][5] = {{1.53, 0.083, 0.046, 1.8, 0.013}, {2.08, 0.159, 0.0, 2.3, 0.0}, {1.49, 0.083, 0.056, 1.4, 0.010}};
+    double fixed = kUs[b][0], store = kUs[b][3], tile = kUs[b][4];
+    const bool wide = p.c_kind != C_BF16;
+    if (p.gate) fixed += 0.65, store = 5.7, tile = 0.016;
+    else if (!w4 && wide) store = 2.5, tile = 0.021;
+    if (!wide && !(p.c_vec && p.N % 4 == 0)) store = 4.5;
+    const double blocks = rounds * (pairs * c.pair[b] + c.block[b] + tile * c.mt * c.nt);
+    const double memory = kUs[b][1] * (weight + a * (a > 4.0 ? tiles_n : fmin(tiles_n, 8.0)));
+    return c.fixed[b] + fixed + hypot(blocks, memory) + kUs[b][2] * weight + store * out;
 }
 
 int skinny_best(const GemmParams& p, bool w4, int num_cus, double* us) {
@@ -256,8 +285,7 @@ int skinny_best(const GemmParams& p, bool w4, int num_cus, double* us) {
         const double ti = skinny_us(p, w4, num_cus, i);
         if (ti < t) t = ti, best = i;
     }
-    // Element-wise stores (odd columns or pitch): 4.5 us a million outputs.
-    *us = t + (p.c_vec && p.N % 4 == 0 ? 0.0 : 4.5e-6 * p.M * p.N);
+    *us = t;
     return best;
 }
 

@@ -383,3 +383,12 @@ def test_gemm_is_small_follows_the_table(lib):
             assert not Q.gemm_is_small(*bad)
     finally:
         Q.gemm_plan_clear()
+
+
+def test_small_problem_rule_leaves_wide_outputs_to_the_persistent_kernel(lib):
+    """Few rows onto very many columns are as fast or faster there (52 x 21192 x
+    2048: 11.7 us against 16.8); a row, a prompt or few columns are not."""
+    for shape in ((52, 21192, 2048), (89, 27504, 5120), (65, 17608, 4608)):
+        assert not Q.gemm_is_small(*shape), shape
+    for shape in ((1, 3072, 3072), (4, 9216, 3072), (256, 3072, 3072), (4173, 64, 3072)):
+        assert Q.gemm_is_small(*shape) and Q.gemm_is_small(*shape, k_tiled=True), shape
