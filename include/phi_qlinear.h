@@ -290,8 +290,10 @@ phi_status phi_hip_q8_linear_kt(phi_stream_t stream, const void* x, int x_dtype,
  * for bit), with the activation scratch q8 written K-tiled where the
  * 272 x 192 plan takes the problem (K % 256 == 0, K <= 16384, 16-byte
  * aligned q8, W rows and C rows): the GEMM then reads A in K-tiled pieces
- * and only the weight's rows are gathered.  Elsewhere it is phi_hip_q8_linear
- * and q8 is row-major.  q8 is scratch either way: callers must not read it. */
+ * and only the weight's rows are gathered.  Elsewhere, and where the
+ * small-problem kernel is faster than that plan (a few hundred rows onto very
+ * many columns), it is phi_hip_q8_linear and q8 is row-major.  q8 is scratch
+ * either way: callers must not read it. */
 phi_status phi_hip_q8_linear_kq(phi_stream_t stream, const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K,
                                 const int8_t* W, int64_t ldw, const float* sW, int sw_scalar, const void* bias,
                                 int bias_dtype, int64_t N, void* C, int c_dtype, int64_t ldc, int8_t* q8, float* s8,

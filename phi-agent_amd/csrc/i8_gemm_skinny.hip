@@ -13,7 +13,7 @@
 // its NW waves split K: wave w takes the 128-column pairs w, w + NW, ... The
 // int32 partial sums are exact in any order and meet in LDS.  That needs no
 // workspace and no second launch, and the tile can be as small as the shape
-// wants: 192 blocks of 16 waves for the example.
+// wants: 192 blocks of 8 waves for the example.
 //
 // A wave streams its operands through LDS of its own (no barriers): the
 // 16-byte chunks of a 128-column pair by direct-to-LDS loads, whole 128-byte

@@ -7,9 +7,10 @@
 // about 4 us and the device a start and a drain, around a prologue that works
 // on 6 KB.  Here every block rotates and quantises the rows itself, into LDS, a
 // group a 16-lane team and under the first loads of its weight rows.  At one
-// row, device time back to back: 3072 -> 3072 7.7 -> 6.6 us, 3072 -> 12288
-// 14.0 -> 11.9, 12288 -> 3072 13.9 -> 12.1; with the host's part 11.1 -> 8.0
-// for the first.  Rows that need a second round of the block's waves run as two
+// row, device time of a graph of calls, the weight in cache (new weights each
+// call): 3072 -> 3072 5.9 -> 4.7 us (7.9 -> 7.2), 3072 -> 12288 10.8 -> 10.0
+// (13.0 -> 12.6), 12288 -> 3072 11.5 -> 9.8 (14.0 -> 12.6); called back to back
+// the first 11.1 -> 7.5.  Rows that need a second round of the block's waves run as two
 // launches: 5 rows of 3072 took 9.7 us here against 7.9.
 #include <atomic>
 

@@ -28,9 +28,13 @@
 // same kernel the activations take: the reference's weight and activation
 // quantisers are one function (quantize_impl_into, core/host/quant.cpp:134-169).
 //
-// All of this runs once per weight load and is bound by HBM at a few bytes per
-// element; the kernels are plain and exact (-ffp-contract=off: every product
-// and sum rounds on its own, as the reference's x86-64 host code does).
+// All of this runs once per weight load and is exact (-ffp-contract=off: every
+// product and sum rounds on its own, as the reference's x86-64 host code does).
+// dequant_rows, convrot_rows and pack_k_tiled are bound by HBM at a few bytes
+// per element, the LoRA fold from a few ranks on by its two roundings an entry
+// (VALU).  dequant_rows, convrot_rows and lora_fold have a form with 16-byte
+// accesses and a plain one, an element a thread, for other alignments and
+// widths (and for small folds); convrot's first is in quant_rotate.hip.
 #include "device_common.hpp"
 #include "i8_gemm.hpp"
 #include "persist_common.hpp"
