@@ -309,11 +309,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void l
 // 100000 x 64 x 4 fp32: 6.3 us, above 16.9; 4352 x 64 x 64 5.7 against 7.1.
 constexpr int LR_TR = 2;
 
-// 64 rows x 64 k of x into registers: lane t holds row t / 4, k 16 (t % 4)..+15.
-template <bool XB>
-__device__ __forceinline__ void fetch_x_tile(const void* __restrict__ x, int64_t ldx, int m0, int M, int k0,
+// 64 rows x 64 k of x into registers: lane t holds row t / 4, k 16 (t % 4)..+15
+// (TAIL: zeros past K, a multiple of 16).
+template <bool XB, bool TAIL>
+__device__ __forceinline__ void fetch_x_tile(const void* __restrict__ x, int64_t ldx, int m0, int M, int K, int k0,
                                              float (&v)[16]) {
     const int row = threadIdx.x >> 2, kk = (threadIdx.x & 3) * 16;
+    if (TAIL && k0 + kk >= K) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = 0.0f;
+        return;
+    }
     const int64_t off = (int64_t)min(m0 + row, M - 1) * ldx + k0 + kk;
     if (XB) {
         const uint4 a = *(const uint4*)((const uint16_t*)x + off), b = *(const uint4*)((const uint16_t*)x + off + 8);
@@ -332,8 +338,9 @@ __device__ __forceinline__ void fetch_x_tile(const void* __restrict__ x, int64_t
     }
 }
 
-// x rows 16-byte aligned, K % 64 == 0.
-template <bool XB>
+// x rows 16-byte aligned, K % 64 == 0, or (TAIL) K % 16 == 0: past K x = 0 and
+// A = -1, as above.  Without it 100000 x 64 x 64 takes 39 us in bf16, with it 44.
+template <bool XB, bool TAIL>
 __global__ __launch_bounds__(256) void lora_down_rows_kernel(const void* __restrict__ x, int64_t ldx,
                                                              const float* __restrict__ A, float* __restrict__ h,
                                                              int M, int K, int R) {
@@ -347,11 +354,12 @@ __global__ __launch_bounds__(256) void lora_down_rows_kernel(const void* __restr
     // holds LR_TR consecutive k of rank l / LPR.  Ranks past R read rank R - 1.
     constexpr int LPR = LD_KC / LR_TR;
     const int at = lane / LPR, ak = (lane % LPR) * LR_TR;
-    const float* arow = A + (int64_t)min(rb + at, R - 1) * K + ak;
+    const float* arow = A + (int64_t)min(rb + at, R - 1) * K;
+    auto fetch_a = [&](int k0) { return !TAIL || k0 + ak < K ? *(const float2*)(arow + k0 + ak) : make_float2(-1.0f, -1.0f); };
     float acc[LR_TR] = {0.0f, 0.0f};
     float xt[16];
-    fetch_x_tile<XB>(x, ldx, m0, M, 0, xt);
-    float2 ta = *(const float2*)arow;
+    fetch_x_tile<XB, TAIL>(x, ldx, m0, M, K, 0, xt);
+    float2 ta = fetch_a(0);
     const int srow = threadIdx.x >> 2, skk = (threadIdx.x & 3) * 16;
     for (int k0 = 0, buf = 0; k0 < K; k0 += LD_KC, buf ^= 1) {
         float* st = sx[buf] + srow * LD_P + skk;
@@ -360,8 +368,8 @@ __global__ __launch_bounds__(256) void lora_down_rows_kernel(const void* __restr
         *(float2*)&sa[buf][wave][at * LD_KC + ak] = ta;
         __syncthreads();
         if (k0 + LD_KC < K) {
-            fetch_x_tile<XB>(x, ldx, m0, M, k0 + LD_KC, xt);
-            ta = *(const float2*)(arow + k0 + LD_KC);
+            fetch_x_tile<XB, TAIL>(x, ldx, m0, M, K, k0 + LD_KC, xt);
+            ta = fetch_a(k0 + LD_KC);
         }
         if (live) {
             const float* xr = sx[buf] + lane * LD_P;
@@ -388,9 +396,10 @@ __global__ __launch_bounds__(256) void lora_down_rows_kernel(const void* __restr
     }
     const int m = m0 + lane;
     if (!live || m >= M) return;
+    const bool pad = TAIL && K % 32 != 0;
 #pragma unroll
     for (int t = 0; t < LR_TR; t++)
-        if (rb + t < R) h[(int64_t)m * R + rb + t] = acc[t];  // K % 32 == 0: no padding
+        if (rb + t < R) h[(int64_t)m * R + rb + t] = pad ? fmaf(0.0f, 0.0f, acc[t]) : acc[t];
 }
 
 template <bool XB, bool VEC, int WR, int RT>
@@ -420,20 +429,26 @@ static hipError_t launch_down_r(hipStream_t stream, const void* x, int64_t ldx, 
                : launch_down<XB, VEC, 4, 2>(stream, x, ldx, A, h, M, K, R);
 }
 
+template <bool XB>
+static hipError_t launch_down_rows(hipStream_t stream, const void* x, int64_t ldx, const float* A, float* h, int M, int K,
+                                   int R) {
+    const dim3 grid((unsigned)(((int64_t)M + 63) / 64), (unsigned)((R + 4 * LR_TR - 1) / (4 * LR_TR)));
+    if (K % LD_KC == 0) hipLaunchKernelGGL((lora_down_rows_kernel<XB, false>), grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
+    else hipLaunchKernelGGL((lora_down_rows_kernel<XB, true>), grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
+    return hipGetLastError();
+}
+
 hipError_t launch_lora_down(hipStream_t stream, const void* x, bool x_bf16, int64_t ldx, const float* A, float* h,
                             int M, int K, int R) {
     const int esz = x_bf16 ? 2 : 4;
-    // One row a lane: a chunk or two of columns, and few ranks of many rows
-    // (measured against the tiles over 1130 sizes: 32760 x 1024 x 4 fp32 21.7
-    // against 26.4 us, 4352 x 64 x 16 4.0 against 5.1; 4352 x 256 x 64 10.7
-    // against 8.5, 32760 x 2048 x 16 80 against 47).
-    if ((K <= 64 || (R <= 16 && K <= 192) || (R <= 8 && M > 16384 && K <= 1024)) && K % LD_KC == 0 &&
-        (uintptr_t)x % 16 == 0 && (ldx * esz) % 16 == 0 && (uintptr_t)A % 16 == 0) {
-        const dim3 grid((unsigned)(((int64_t)M + 63) / 64), (unsigned)((R + 4 * LR_TR - 1) / (4 * LR_TR)));
-        if (x_bf16) hipLaunchKernelGGL(lora_down_rows_kernel<true>, grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
-        else hipLaunchKernelGGL(lora_down_rows_kernel<false>, grid, dim3(256), 0, stream, x, ldx, A, h, M, K, R);
-        return hipGetLastError();
-    }
+    // One row a lane: few columns, and few ranks of many rows (measured against
+    // the tiles over 1350 sizes: 32760 x 1024 x 4 fp32 21.7 against 26.4 us, 4352
+    // x 64 x 16 4.0 against 5.1; 4352 x 256 x 64 10.7 against 8.5, 32760 x 2048 x
+    // 16 80 against 47).
+    if ((K <= 64 || (K <= 192 && (R <= 16 || M <= 1024)) || (R <= 8 && M > 16384 && K <= 1024)) && K % 16 == 0 &&
+        (uintptr_t)x % 16 == 0 && (ldx * esz) % 16 == 0 && (uintptr_t)A % 16 == 0)
+        return x_bf16 ? launch_down_rows<true>(stream, x, ldx, A, h, M, K, R)
+                      : launch_down_rows<false>(stream, x, ldx, A, h, M, K, R);
     const bool vec = K % 4 == 0 && ldx % 4 == 0 && (uintptr_t)x % (4 * esz) == 0 && (uintptr_t)A % 16 == 0;
     if (x_bf16) return vec ? launch_down_r<true, true>(stream, x, ldx, A, h, M, K, R)
                            : launch_down_r<true, false>(stream, x, ldx, A, h, M, K, R);

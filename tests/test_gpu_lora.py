@@ -172,7 +172,7 @@ def test_lora_tiles_bit_exact(dev, orc, cdt, M, K, N, R):
 
 
 @pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("M,K,R", [(1, 64, 1), (65, 64, 17), (129, 64, 130), (64, 128, 16), (70, 192, 9), (70, 192, 17),
+@pytest.mark.parametrize("M,K,R", [(1, 64, 1), (65, 64, 17), (129, 64, 130), (70, 16, 5), (70, 32, 40), (70, 48, 33), (70, 144, 16), (64, 128, 16), (70, 192, 9), (1024, 192, 17), (1025, 192, 17),
                                    (16384, 256, 8), (16385, 256, 8), (16385, 1024, 3), (16385, 256, 9)])
 def test_lora_down_one_row_a_lane(dev, orc, xdt, M, K, R):
     """Both sides of the lines between the chains of one row a lane and the
