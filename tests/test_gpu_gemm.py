@@ -361,3 +361,37 @@ def test_odd_columns_over_several_tiles(dev, monkeypatch, out, M, N, K):
             got.append(Q.i8_gemm(A, B, sA, sB, bias, out_dtype=out))
             torch.cuda.synchronize()
         assert torch.equal(got[0], got[1])
+
+
+def _graph_us(fn, calls=10):
+    fn()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for _ in range(calls):
+            fn()
+    g.replay()
+    best = float("inf")
+    for _ in range(7):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        g.replay()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / calls)
+    return best
+
+
+# Deep problems of half a round of 256 x 256 tiles or more, K in no pairs of
+# 128: the small-problem kernel took 1.1 to 1.2 times the tiles' time.
+@pytest.mark.parametrize("M,N,K,out", [(2913, 3124, 13696, torch.int32), (9987, 1776, 11904, torch.bfloat16)])
+def test_deep_tiles_stay_off_the_small_problem_kernel(dev, monkeypatch, M, N, K, out):
+    A, B = synth.int8_weight(M, K, seed=M, device=dev), synth.int8_weight(N, K, seed=N + 1, device=dev)
+    sA, sB = torch.rand(M, device=dev), torch.rand(N, device=dev)
+    us, C = {}, torch.empty((M, N), dtype=out, device=dev)
+    for skinny in ("off", "", "off", ""):
+        monkeypatch.delenv("PHI_GEMM_SKINNY", raising=False)
+        if skinny:
+            monkeypatch.setenv("PHI_GEMM_SKINNY", skinny)
+        us[skinny] = min(us.get(skinny, 1e9), _graph_us(lambda: Q.i8_gemm(A, B, sA, sB, C=C)))
+    assert us[""] < 1.06 * us["off"], us
