@@ -288,15 +288,23 @@ double persist_us(const phi_dev::GemmParams& p, bool w4, int G) {
 }
 
 // The same of the register-staged tile kernels (gemm_kernel_for, gemm_cfg_for).
-// 256 x 256 tiles: 694 shapes with 128 of them or more, rms error 6 to 8 %, one
-// 64-deep step 0.71 us.  Fewer keep the least that 128 x 128 tiles take (as low
-// as a quarter of the time of short problems, up to 13 % over at long ones).
+// 256 x 256 tiles: 1222 shapes with 128 of them or more, rms error 7 %.  Fewer
+// keep the least that 128 x 128 tiles take (as low as a quarter of the time of
+// short problems, up to 13 % over at long ones).
 double tile_us(const phi_dev::GemmParams& p, int G) {
     const double t256 = ceil(p.M / 256.0) * ceil(p.N / 256.0), steps = (p.K + 63) / 64;
     if (t256 < 128) return 4.0 + 0.40 * fmax(1.0, ceil(p.M / 128.0) * ceil(p.N / 128.0) / (2 * G)) * steps;
-    const bool i32 = p.c_kind == phi_dev::C_I32;
-    const double out = 1e-6 * p.M * p.N * (!p.c_vec ? 2.56 : p.c_kind == phi_dev::C_BF16 ? 0.61 : 0.92);
-    return 4.0 + ceil(t256 / G) * ((i32 ? 0.1 : 5.0) + 0.71 * steps) + out;
+    const double out = (p.c_kind == phi_dev::C_BF16 ? 0.3 : 0.42) + (p.c_vec ? 0.0 : 2.0);
+    return 3.8 + ceil(t256 / G) * ((p.c_kind == phi_dev::C_I32 ? 6.9 : 11.2) + 0.45 * steps) + 21.6 * lds_gb(p) + out * 1e-6 * p.M * p.N;
+}
+
+// The same of the pipeline with the element-wise epilogue, over 2066 shapes (6
+// %).  Against the register-staged tiles: 4096 x 4101 x 3072 in bf16 139 -> 94
+// us, 8000 x 11645 x 1024 in fp32 384 -> 261, 2000 x 1001 x 2048 26 -> 17
+// (whole pieces take 58, 200 and 9).
+double loose_us(const phi_dev::GemmParams& p, int G) {
+    const double rounds = square_plan_cost(p.M, p.N, G);
+    return 2.6 + rounds * (19.0 + 0.546 * (p.K / 64)) + 0.016e-6 * ((double)p.N + p.M) * p.K + 15.6 * lds_gb(p) + 0.556e-6 * p.M * p.N;
 }
 
 // The same of W4A8 with per-group tables: expanded once into a workspace, in
@@ -328,25 +336,30 @@ int skinny_choice(const phi_dev::GemmParams& p, bool w4, int G, double other_us)
 
 // Whether a problem the persistent kernel refuses only for its output (pieces
 // or rows that are no whole 16 bytes) runs on the pipeline with the
-// element-wise epilogue.  Between one and two rounds of 128 x 128 tiles the
-// register-staged kernel keeps it: two of its blocks share a CU, and the two
-// take the same time (1023 x 4101 x 3072: 41 us each; 1358 x 4391 x 2048: 33
-// against 34).  PHI_GEMM_LOOSE=0 keeps the pipeline out, 1 takes both.
+// element-wise epilogue.  The register-staged tiles keep
+//   - up to one round of 256 x 256 tiles that is less than half full, but over
+//     one round of 128 x 128 tiles: two of its blocks share a CU, and the two
+//     take the same time (1023 x 4101 x 3072: 41 us each; 1358 x 4391 x 2048:
+//     33 against 34);
+//   - rows whose pitch is whole pieces of four columns (c_vec), which they
+//     store as pieces: 16287 x 2628 x 256 in bf16 61 us against 89 here, 29774
+//     x 2580 x 1024 166 against 201, 30620 x 1701 x 256 in int32 58 against 114.
+//     Of those the pipeline has only what fits one round of 128 x 128 tiles (125
+//     x 19420 x 4096 27 us against 42; int32 needs 1024 deep for it: 1572 x 237
+//     x 256 11 against 8.5, 612 x 2605 x 1024 equal), and what the models give
+//     it: mostly a second round of 256 x 256 tiles that would be a few tiles,
+//     which its 128 x 128 tiles shorten (822 x 17708 x 7424 140 against 176).
+//     Of 1029 shapes one took over 4 % more than on the staged tiles (9 %).
+// PHI_GEMM_LOOSE=0 keeps the pipeline out, 1 takes all of it.
 bool loose_ok(const phi_dev::GemmParams& p, bool pok, bool staged_ok) {
     const int64_t lim = (int64_t)1 << 23;
+    const int G = num_cus();
+    if (pok || !staged_ok || p.K % 256 != 0 || p.lda >= lim || p.ldb >= lim || p.ldc >= lim / 4 || getenv("PHI_GEMM_KERNEL")) return false;
+    const int forced = phi_dev::env_switch("PHI_GEMM_LOOSE", -1, 0, 1);
+    if (forced >= 0) return forced;
     const int64_t big = ((int64_t)p.M + 255) / 256 * ((p.N + 255) / 256), small = ((int64_t)p.M + 127) / 128 * ((p.N + 127) / 128);
-    if (big < 128 && small > num_cus() && !phi_dev::env_switch("PHI_GEMM_LOOSE", 0, 0, 1)) return false;
-    return !pok && staged_ok && p.K % 256 == 0 && p.lda < lim && p.ldb < lim && p.ldc < lim / 4 && !getenv("PHI_GEMM_KERNEL") &&
-           phi_dev::env_switch("PHI_GEMM_LOOSE", 1, 0, 1);
-}
-
-// The same as persist_us for it.  Against
-// the register-staged tiles: 4096 x 4101 x 3072 in bf16 139 -> 94 us, 8000 x
-// 11645 x 1024 in fp32 384 -> 261, 2000 x 1001 x 2048 26 -> 17 (whole pieces
-// take 58, 200 and 9).
-double loose_us(const phi_dev::GemmParams& p, int G) {
-    const double rounds = square_plan_cost(p.M, p.N, G);
-    return 3.6 + rounds * (12.9 + 0.508 * (p.K / 64)) + 0.01e-6 * ((double)p.N + p.M) * p.K + 33.7 * lds_gb(p) + 1.0e-6 * p.M * p.N;
+    if (small <= G) return !(p.c_vec && p.c_kind == phi_dev::C_I32) || p.K >= 1024;
+    return big >= 128 && (!p.c_vec || loose_us(p, G) < 0.97 * tile_us(p, G));
 }
 
 // Whether a tuning-table entry says how the persistent kernel runs (and not
